@@ -24,6 +24,16 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "slow: takes more than a few seconds on the CPU")
 
 
+def pytest_collection_modifyitems(items):
+    """The facade test compiles the reference's sources; a reference folder
+    that exists but holds none is the same as an absent one."""
+    if os.path.isfile("/root/reference/sim.cpp"):
+        return
+    for it in items:
+        if it.name == "test_reference_driver_compiles_against_facade":
+            it.add_marker(pytest.mark.skip(reason="reference sources absent"))
+
+
 @pytest.fixture(scope="session", params=["mfma", "valu"])
 def ctx(request):
     """A GPU context per lead-contraction path: every GPU test runs on both
