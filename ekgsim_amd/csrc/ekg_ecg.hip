@@ -1180,206 +1180,340 @@ __global__ void ecg_reduce_kernel(const HeartDev* __restrict__ hearts, const Req
 // Activation classes
 // ---------------------------------------------------------------------------
 
-constexpr int CC_THREADS = 256;
-
-// Class windows: one block per (piece of a class window, request).  Every
-// voxel of a class has the same AP, so only the sum of the class's G rows is
-// needed, and by regrouping the dipoles per cell it is
+// Class boxes.  Every voxel of a class has the same AP, so only the sum of
+// the class's G rows is needed, and by regrouping the dipoles per cell it is
 //   sum_u G(u) = sum_w s(w) (e(w) . D(w))
 // over the cells w with a non-zero integer vector D(w) for the class
-// (host-built per neighbourhood; cells inside the class cancel).  With
-// e = p - c (c the cell's coordinate + 1) this is linear in the electrode p:
-//   sum_w s(w) (e . D) = p . T + T3,  T_c = sum_w s(w) D_c(w),  T3 = sum_w s(w) K(w),
-// K = -D . c.  A cell borders several classes, so the host lists each cell
-// once per window of CLASS_WINDOW classes (an entry) with its D and K for
-// each class of the window, and the weight s(w) is evaluated once per entry
-// and lead.  The squared distance and the products run on
-// v_mfma_f64_4x4x4f64 (4 blocks of 4 x 4 x 4):
-//  1. |e|^2 = |p|^2 - 2 p . c + |c|^2 as an FP64 matrix product: rows are the
-//     16 entries of a group (4 per block), columns the 4 leads of a group, the
-//     inner dimension {c_z, c_y, c_x, 1} x {-2 p_z, -2 p_y, -2 p_x, |p|^2},
-//     with |c|^2 (exact) as the accumulator input;
-//  2. s = rsq(|e|^2 rounded to FP32)^3 in FP32 -- the chunk kernel's weight:
-//     it rounds its own FP64 |e|^2 (from the exact FP64 offsets, a
-//     neighbour's from the voxel's |e|^2 and dipole sum) the same way, so the
-//     two kernels give a cell the same weight except where the two FP64
-//     values (both within ~1e-14 relative of |e|^2) straddle an FP32
-//     rounding boundary;
-//  3. for each class i of the group's mask, T_i += s x {D_z, D_y, D_x, K}_i:
-//     rows the leads, inner dimension the entries, one accumulator per class
-//     of the window.
-// gfx950 lane layout (checked by a one-hot probe): A(block, row, k) in lane
-// 16k + 4 block + row, B(block, k, col) in lane 16k + 4 block + col,
-// D(block, row, col) in lane 16 row + 4 block + col.  Product 1's result for
-// (entry r of block b, lead col) lands in lane 16r + 4b + col, which is where
-// product 3 takes its operand (block b, lead row, entry k): so a lane owns one
-// entry of each group of 16 and one lead of each group of 4 throughout, and
-// feeds product 1 coordinate (lane >> 4) of entry (b, lane & 3).  The host
-// stores those per-lane operands of every group lane-major, so a lane loads
-// coalesced words and converts them, with no index arithmetic or unpacking.
-// Each wave takes groups of the piece strided over the waves, the blocks'
-// partial sums are added in block order, the waves' in wave order, and
-// sums[(c_off + n_chunks + p CLASS_WINDOW + i)*3*LP] receives the piece's
-// {sum G, P' sum G, Q' sum G} of class i of its window, with the class's
-// P' = k2(1-k3) e^{(k4+k5)(a - t0)} and Q' = k2 k3 e^{k5 (a - t0)} (zero for
-// a class past the heart's last).
-template <int LP>
-__global__ __launch_bounds__(CC_THREADS) void ecg_class_window_kernel(
-    const HeartDev* __restrict__ hearts, const ReqDev* __restrict__ reqs, const int4* __restrict__ runs,
-    const int64_t* __restrict__ run_start, int n_runs, const double* __restrict__ lead_pos,
-    const double* __restrict__ layer_k, double* __restrict__ sums)
+// (host-built per neighbourhood; cells inside the class cancel), s = |e|^-3,
+// e = p - c (c the cell's coordinate + 1).  About c0, a point of the cell's box,
+// this is
+//   (p - c0) . T + T3,  T_c = sum_w s(w) D_c(w),  T3 = sum_w s(w) K(w),
+// K = -D . (c - c0), c0 the box's first cell: D and K fit in a byte.
+//
+// What bounds it: vector issue, mostly the weights' (about 34 cycles per 64
+// weights: 8 for the reciprocal square root, 8 each for |e|^2 with its
+// rounding, the conversion with the offset and the byte transposition).  So every
+// cell is evaluated once per lead, whatever number of classes it borders (4.5
+// on the 128^3 heart of integer delays), and the sums run on the int8 matrix
+// cores, where a class costs little:
+//  * A box is 4 x 8 x 8 cells, four sub-bricks of 4^3 whose 64 cells are the
+//    inner dimension of v_mfma_i32_16x16x64_i8: lane = 16 z + lead column,
+//    byte 4 y + x.  In the dense sub-brick |e|^2 = X[x] + Y[y] (Y with the
+//    lane's z), one FP64 add per cell; cells without dipoles have zero
+//    coefficients, rows of 16 cells without any are skipped.
+//  * The weight is the chunk kernel's FP32 one, s = rsq(|e|^2 rounded to FP32)^3,
+//    with the electrode's distances scaled by a power of two so that the
+//    largest weight lies in [2^27, 2^30].  Unless the electrode is near (about 8
+//    voxels), the smallest is at least 2^23, so the FP32 weight is an integer
+//    and its conversion exact; near boxes take further passes over the
+//    fraction that is left (x 2^30, again exact in FP32) until the smallest
+//    weight is covered too.
+//  * The integer's four bytes, each less 128 (the accumulators start at 128 times
+//    the coefficient sums), are one operand of four products, 16 leads wide; the
+//    other holds 4 classes x {D_z, D_y, D_x, K} of the sub-brick's 64 cells.  The
+//    sums are exact integers; only the flush, once per box and 4 classes, rounds (FP64).
+//  * Rows of 16 leads are filled across the requests of a heart, so no lead slot
+//    is idle whatever the lead count.
+// A block of 4 waves takes one region (a run of boxes with at most CB_SLOTS
+// classes) for 16 leads; wave w takes boxes w, w + 4, ... (ordered by the host so
+// that the waves' work is equal) and adds their class sums into its own
+// LDS rows in order, then the waves' rows are added in wave order into
+// gsum[line of (region, class)][lead].  The cut into regions and the order
+// depend on the heart only, so a request's bits do not depend on its batch.
+// Measured per 256 x 12 launch on the 128^3 heart: 0.83 ms (vector instructions
+// 0.52 and matrix products 0.15 of it), against 1.37 ms with the weights
+// evaluated per window of six classes and FP64 products; 16 x 12 on the 256^3 heart
+// 0.35 against 0.69 ms.  Regions of 64 classes instead of 96: 0.97 ms (a block's
+// start and end weigh more); boxes in grid order within a region: 0.85 ms; two
+// waves a SIMD 0.98 ms.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// Byte transposition: the words of cells x = 0 .. 3 to the words of the four
+// bytes, each byte less 128.
+__device__ __forceinline__ void limbs4(const int q[4], int out[4])
 {
-    constexpr int NG = LP / 4;                 // groups of 4 leads
-    constexpr int NW = CC_THREADS / 64;
-    constexpr int CW = CLASS_WINDOW;
-    __shared__ double s_t[CW][NW][LP][4];
+    const unsigned a = __builtin_amdgcn_perm(q[1], q[0], 0x05010400u), b = __builtin_amdgcn_perm(q[1], q[0], 0x07030602u),
+                   c = __builtin_amdgcn_perm(q[3], q[2], 0x05010400u), d = __builtin_amdgcn_perm(q[3], q[2], 0x07030602u);
+    out[0] = (int)(__builtin_amdgcn_perm(c, a, 0x05040100u) ^ 0x80808080u);
+    out[1] = (int)(__builtin_amdgcn_perm(c, a, 0x07060302u) ^ 0x80808080u);
+    out[2] = (int)(__builtin_amdgcn_perm(d, b, 0x05040100u) ^ 0x80808080u);
+    out[3] = (int)(__builtin_amdgcn_perm(d, b, 0x07060302u) ^ 0x80808080u);
+}
+
+// FP32 to int32 toward zero, saturating, NaN to 0 (the instruction's own rule).
+__device__ __forceinline__ int cvt_i32(float x)
+{
+    int r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
+// Power-of-two scale of a lead's distances to a box of cells, first cell at
+// the electrode's offset -(q), half extents h: distances x 2^-m put the
+// nearest into [2^-10, 2^-9), the largest weight into [2^27, 2^30].  exact:
+// the smallest weight is at least 2^23 (the farthest cell's scaled |e|^2 at most
+// 2^(-46/3)), so every FP32 weight is an integer, and the electrode is at least 2
+// voxels off, where FP32 distances are good to the margin taken.  Electrodes
+// without FP32 distances (above 1e15, or not finite) have weight 0 or a
+// non-finite flush factor, whatever the scale.
+struct ScaleRange {
+    float df;
+    int m;
+    bool exact;
+};
+__device__ __forceinline__ ScaleRange scale_range(float qz, float qy, float qx, float hz, float hy, float hx)
+{
+    const float az = fabsf(qz - hz), ay = fabsf(qy - hy), ax = fabsf(qx - hx);
+    const float nz = fmaxf(az - hz, 0.0f), ny = fmaxf(ay - hy, 0.0f), nx = fmaxf(ax - hx, 0.0f);
+    const float fz = az + hz, fy = ay + hy, fx = ax + hx;
+    const float dn = 0.9999f * __builtin_fmaf(nx, nx, __builtin_fmaf(ny, ny, nz * nz));
+    ScaleRange r;
+    r.df = 1.0001f * __builtin_fmaf(fx, fx, __builtin_fmaf(fy, fy, fz * fz));
+    r.m = ((int)((__float_as_uint(dn) >> 23) & 255u) - 127 + 20) >> 1;
+    r.exact = !(dn <= 1e30f) || (dn >= 4.0f && __builtin_ldexpf(r.df, -2 * r.m) <= 2.4e-5f);
+    return r;
+}
+
+__global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
+    const HeartDev* __restrict__ hearts, const ClassSeg* __restrict__ segs, int n_segs, const int* __restrict__ rowpos,
+    const double* __restrict__ lead_pos, double* __restrict__ gsum)
+{
+    __shared__ double s_acc[CB_WAVES][CB_SLOTS + 1][16];  // last row: classes past a tile's end
+    __shared__ i32x4 s_init[CB_WAVES][64];
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    // Piece-major within each run of requests of one heart (a run
-    // {first request, requests, pieces}): the requests of a piece run back to
-    // back and read its groups from L2 (blocks go round-robin over the XCDs,
-    // so each XCD fetches a piece once per run).
-    const int u = find_req(run_start, n_runs, blockIdx.x);
-    const int4 run = runs[u];
-    const int local = (int)(blockIdx.x - run_start[u]);
-    const int k = local / run.y, r = run.x + (local - k * run.y);
-    const ReqDev& R = reqs[r];
-    const HeartDev& H = hearts[R.heart];
-    const int4 pc4 = H.cpieces[k];
-    const int pw = __builtin_amdgcn_readfirstlane(pc4.x), g0 = __builtin_amdgcn_readfirstlane(pc4.y),
-              g1 = __builtin_amdgcn_readfirstlane(pc4.z);
-    const int rc = lane & 3;                                  // lead of a group (and product-3 column)
-    const int kq = lane >> 4;                                 // product-1 inner index: coordinate kq
-    // product-1 right operand: {-2 p_z, -2 p_y, -2 p_x, |p|^2} of the lane's
-    // leads 4g + rc (leads past the request's count repeat lead 0; their sums
-    // are zeroed)
-    double pe[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        const int i = 4 * g + rc < R.L ? 4 * g + rc : 0;
-        const double* p = lead_pos + R.pos_off + 3 * i;
-        const double pp = __builtin_fma(p[2], p[2], __builtin_fma(p[1], p[1], p[0] * p[0]));
-        pe[g] = kq < 3 ? -2.0 * p[kq < 3 ? kq : 0] : pp;
+    const int64_t blk = segs[0].block0 + blockIdx.x;
+    int u = 0;
+    for (int hi = n_segs; hi - u > 1;) {
+        const int mid = (u + hi) >> 1;
+        if (segs[mid].block0 <= blk)
+            u = mid;
+        else
+            hi = mid;
     }
-    double acc[CW][NG];
-#pragma unroll
-    for (int i = 0; i < CW; ++i)
-#pragma unroll
-        for (int g = 0; g < NG; ++g) acc[i][g] = 0.0;
-    // Each group's rows and class mask are wave-uniform: read through the
-    // constant address space they become scalar loads, and the group's rows
-    // through the global one take a scalar base and the lane's offset, so
-    // neither needs vector address arithmetic.
-    using ci64 = __attribute__((address_space(4))) const long long;
-    ci64* const crow = (ci64*)H.crow;
-    for (int q = g0 + w; q < g1; q += NW) {
-        const long long cr = crow[q];  // {first row, class mask}
-        const int row = (int)(cr & 0xffffffffLL), mask = (int)(cr >> 32);
-        // the group's rows as a buffer resource: the lane's offset is a
-        // fixed vector operand and each row's offset a scalar one (reads
-        // past the group's rows would return 0, never fault)
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(H.cgrp + (int64_t)64 * row), 0, 256 * (2 + __builtin_popcount(mask)), 0x00020000);
-        const int lo = 4 * lane;
-        // product-1 left operand (coordinate kq of entry 4 block + rc, or 1)
-        // and |c|^2 of entry 4 block + kq
-        const double av = (double)__int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, lo, 0, 0));
-        const double cc = (double)__int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, lo, 256, 0));
-        float bf[CW];
-#pragma unroll
-        for (int i = 0, n = 2; i < CW; ++i)
-            if ((mask >> i) & 1) bf[i] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, lo, 256 * n++, 0));
-        // A wave past its loads takes issue priority for the products and
-        // weights of the group, and gives it back once its next loads are
-        // due, so that the waves of a SIMD spread over the loop instead of
-        // waiting on their loads together (measured: 1.0% per step).
-        __builtin_amdgcn_s_setprio(1);
-        double sw[NG];
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const double e2 = __builtin_amdgcn_mfma_f64_4x4x4f64(av, pe[g], cc, 0, 0, 0);
-            const float rr = __builtin_amdgcn_rsqf((float)e2);
-            sw[g] = (double)(rr * rr * rr);
-        }
-#pragma unroll
-        for (int i = 0; i < CW; ++i)
-            if ((mask >> i) & 1) {
-                // product-3 right operand: coefficient rc of entry 4 block + kq for class i
-                const double bv = (double)bf[i];
-#pragma unroll
-                for (int g = 0; g < NG; ++g) acc[i][g] = __builtin_amdgcn_mfma_f64_4x4x4f64(sw[g], bv, acc[i][g], 0, 0, 0);
-            }
-        __builtin_amdgcn_s_setprio(0);
+    const ClassSeg sg = segs[u];
+    // Blocks go round-robin over the 8 XCDs: eight regions at a time, region 8 g + x
+    // on XCD x with all its rows of 16 leads back to back, so that each region's
+    // coefficients are fetched into one L2.  A block takes sg.per rows of a
+    // region in turn (the chain of loads that starts a block, paid once).
+    const int local = (int)(blk - sg.block0), n8 = sg.n_regions >> 3, ns = (sg.n_rg + sg.per - 1) / sg.per;
+    int k, rg;
+    if (local < 8 * n8 * ns) {
+        const int q = local >> 3;
+        k = 8 * (q / ns) + (local & 7);
+        rg = q % ns * sg.per;
+    } else {
+        const int q = local - 8 * n8 * ns;
+        k = 8 * n8 + q / ns;
+        rg = q % ns * sg.per;
     }
-    // acc[i][g] in lane 16 row + 4 block + col: lead 4g + row, coefficient
-    // col, this wave's entries of one block; the four blocks in order
-    const int base = lane & ~12;
-#pragma unroll
-    for (int i = 0; i < CW; ++i)
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const double v0 = __shfl(acc[i][g], base), v1 = __shfl(acc[i][g], base | 4),
-                         v2 = __shfl(acc[i][g], base | 8), v3 = __shfl(acc[i][g], base | 12);
-            if ((lane & 12) == 0) s_t[i][w][4 * g + (lane >> 4)][lane & 3] = ((v0 + v1) + v2) + v3;
+    const int rg_end = rg + sg.per < sg.n_rg ? rg + sg.per : sg.n_rg;
+    const HeartDev& H = hearts[sg.heart];
+    using ci32x4 = __attribute__((address_space(4))) const i32x4;
+    using gi32x4 = __attribute__((address_space(1))) const i32x4;
+    using gint = __attribute__((address_space(1))) const int;
+    using gf64 = __attribute__((address_space(1))) const double;
+    const i32x4 reg = ((ci32x4*)H.cregion)[2 * k];      // {first box, end box, first line, lines}
+    const i32x4 ext = ((ci32x4*)H.cregion)[2 * k + 1];  // {z0 | z1 << 16, y0 | y1 << 16, x0 | x1 << 16, 0}: cells + 1
+    gi32x4* const pkt = (gi32x4*)H.cbox + lane;
+    gi32x4* const ini = (gi32x4*)H.cinit + lane;
+    const char* const coef = (const char*)H.ccoef;
+    const int n_lines = H.n_lines;
+    const int zq = lane >> 4;
+    // electrode position offset of the lane's lead
+    int po = ((gint*)rowpos)[16 * (sg.rg0 + rg) + (lane & 15)];
+    for (; rg < rg_end; ++rg) {
+        const double p0 = ((gf64*)lead_pos)[po], p1 = ((gf64*)lead_pos)[po + 1], p2 = ((gf64*)lead_pos)[po + 2];
+        if (rg + 1 < rg_end) po = ((gint*)rowpos)[16 * (sg.rg0 + rg + 1) + (lane & 15)];
+        for (int i = lane; i < (CB_SLOTS + 1) * 16; i += 64) (&s_acc[w][0][0])[i] = 0.0;
+
+        // One scale for the whole region where every lead of the row allows it
+        // (most regions: a lead at least about 10 voxels off), else per box.
+        ScaleRange rr = scale_range((float)(p0 - (double)(ext.x & 0xffff)), (float)(p1 - (double)(ext.y & 0xffff)),
+                                    (float)(p2 - (double)(ext.z & 0xffff)), 0.5f * (float)((ext.x >> 16) - (ext.x & 0xffff)),
+                                    0.5f * (float)((ext.y >> 16) - (ext.y & 0xffff)),
+                                    0.5f * (float)((ext.z >> 16) - (ext.z & 0xffff)));
+        const bool per_box = __any(!rr.exact);
+        int m = rr.m;
+
+        // Every box's records are read a box ahead, as one packet of 16 bytes a lane
+        // (tile records in lanes 0 .. 15, the box's in 16 and 17) and one of the
+        // tiles' accumulator starts, so that no box waits for its own.
+        const int b0 = reg.x + w;
+        i32x4 npk = i32x4{0, 0, 0, 0}, nin = npk;
+        if (b0 < reg.y) {
+            npk = pkt[(int64_t)64 * b0];
+            nin = ini[(int64_t)64 * b0];
         }
-    __syncthreads();
-    for (int u = t; u < CW * LP; u += CC_THREADS) {
-        const int i = u / LP, ld = u - i * LP;
-        const int kc = CW * pw + i;
-        double T[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            T[c] = 0.0;
-#pragma unroll
-            for (int ww = 0; ww < NW; ++ww) T[c] += s_t[i][ww][ld][c];
-        }
-        double sg = 0.0, pp = 0.0, qq = 0.0;
-        if (kc < H.n_classes) {
-            if (ld < R.L) {
-                const double* p = lead_pos + R.pos_off + 3 * ld;
-                sg = __builtin_fma(p[2], T[2], __builtin_fma(p[1], T[1], __builtin_fma(p[0], T[0], T[3])));
+        for (int b = b0; b < reg.y; b += CB_WAVES) {
+            const i32x4 tr = npk;  // lane l < 16: tile l {sub-bricks, 4 slot bytes, first block, 0}
+            s_init[w][lane] = nin;
+            // lane 16: {tiles, rows (4 sub-brick + y) in use, 0, 0}; lane 17: first cell + 1
+            const int nt = __builtin_amdgcn_readlane(tr.x, 16), rows = __builtin_amdgcn_readlane(tr.y, 16);
+            // electrode relative to the box's first cell
+            double qz = p0 - (double)__builtin_amdgcn_readlane(tr.x, 17), qy = p1 - (double)__builtin_amdgcn_readlane(tr.y, 17),
+                   qx = p2 - (double)__builtin_amdgcn_readlane(tr.z, 17);
+            const int bn = b + CB_WAVES < reg.y ? b + CB_WAVES : b;
+            npk = pkt[(int64_t)64 * bn];
+            nin = ini[(int64_t)64 * bn];
+            int np = 1;
+            bool hot = false;
+            if (per_box) {
+                const ScaleRange br = scale_range((float)qz, (float)qy, (float)qx, 1.5f, 3.5f, 3.5f);
+                m = br.m;
+                hot = __any(!br.exact);
+                if (!br.exact) {
+                    // the nearest cell itself, in FP64
+                    const double rz = fmin(fmax(rint(qz), 0.0), 3.0), ry = fmin(fmax(rint(qy), 0.0), 7.0),
+                                 rx = fmin(fmax(rint(qx), 0.0), 7.0);
+                    const double d2 = fmax((qz - rz) * (qz - rz) + (qy - ry) * (qy - ry) + (qx - rx) * (qx - rx), 0x1p-84);
+                    m = ((int)((__double_as_longlong(d2) >> 52) & 2047) - 1023 + 20) >> 1;
+                    // passes of 30 bits until the smallest weight's 24 bits are
+                    // covered: log2 s >= -1.5 (floor(log2 |e|^2) + 1)
+                    const int ef = (int)((__float_as_uint(br.df) >> 23) & 255u) - 127 - 2 * m + 1;
+                    np = 1 + (23 + ((3 * ef + 1) >> 1) + 29) / 30;
+                }
             }
-            const int l = H.classes[kc].x;
-            const double* kk = layer_k + R.k_off + 9 * (l - 1);
-            const double da = H.class_a[kc] - H.layer_t0[l];
-            pp = kk[2] * (1.0 - kk[3]) * exp((kk[4] + kk[5]) * da);
-            qq = kk[2] * kk[3] * exp(kk[5] * da);
+            const double st = __longlong_as_double((long long)(1023 - m) << 52);  // 2^-m
+            double sc = __longlong_as_double((long long)(1023 - 3 * m) << 52);
+            for (int pass = 0;; ++pass) {
+                // |e|^2 x 4^-m = X[x] + Y[y], formed in each pass (the pin keeps them
+                // out of the registers of the tile loop below)
+                asm volatile("" : "+v"(qz), "+v"(qy), "+v"(qx));
+                double X[8], Y[8];
+                const double sz = qz * st, sy = qy * st, sx = qx * st;
+                const double tz = __builtin_fma((double)-zq, st, sz), Z = tz * tz;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const double tx = __builtin_fma((double)-i, st, sx), ty = __builtin_fma((double)-i, st, sy);
+                    X[i] = tx * tx;
+                    Y[i] = __builtin_fma(ty, ty, Z);
+                }
+                // the first tile's operands, on their way during the weights
+                int ti = 0, mask = __builtin_amdgcn_readlane(tr.x, 0);
+                i32x4 A[4];
+                auto load_tile = [&]() {
+                    // an absent sub-brick's load has no records and returns zeros: the
+                    // same number of loads whatever the mask, so that none waits for another
+                    const char* cb = coef + (int64_t)1024 * __builtin_amdgcn_readlane(tr.z, ti & 15);
+#pragma unroll
+                    for (int sb = 0; sb < 4; ++sb) {
+                        const int n = (mask << (10 - sb)) & 1024;
+                        A[sb] = __builtin_bit_cast(
+                            i32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                       __builtin_amdgcn_make_buffer_rsrc((void*)cb, 0, n, 0x00020000), 16 * lane, 0, 0));
+                        cb += n;
+                    }
+                };
+                load_tile();
+                bool bad = false;
+                i32x4 W[4][4];  // [sub-brick][limb]: bytes 4 y + x
+#pragma unroll
+                for (int sb = 0; sb < 4; ++sb) {
+                    const unsigned cm = hot ? (unsigned)(H.cmask[4 * b + sb] >> (16 * zq)) : 0u;
+#pragma unroll
+                    for (int y = 0; y < 4; ++y) {
+                        if (!((rows >> (4 * sb + y)) & 1)) continue;
+                        float s[4];
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            const float r = __builtin_amdgcn_rsqf((float)(X[4 * (sb & 1) + x] + Y[4 * (sb >> 1) + y]));
+                            s[x] = r * r * r;
+                        }
+                        if (hot) {
+                            // an electrode on the centre of a cell with dipoles: its sums are not finite
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) bad |= ((cm >> (4 * y + x)) & 1u) && s[x] == __builtin_inff();
+#pragma unroll 1
+                            for (int h = 0; h < pass; ++h)
+#pragma unroll
+                                for (int x = 0; x < 4; ++x) s[x] = __builtin_amdgcn_fractf(s[x]) * 0x1p30f;
+                        }
+                        const int q[4] = {cvt_i32(s[0]), cvt_i32(s[1]), cvt_i32(s[2]), cvt_i32(s[3])};
+                        int o4[4];
+                        limbs4(q, o4);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) W[sb][j][y] = o4[j];
+                    }
+                }
+                if (hot) {
+                    const int any4 = (int)bad | __shfl_xor((int)bad, 16, 64);
+                    if (any4 | __shfl_xor(any4, 32, 64)) sc = __builtin_nan("");
+                }
+                const double cz = qz * sc, cy = qy * sc, cx = qx * sc;
+                for (;;) {
+                    const i32x4 c0 = s_init[w][4 * (ti & 15) + zq];
+                    i32x4 a0 = c0, a1 = c0, a2 = c0, a3 = c0;
+#pragma unroll
+                    for (int sb = 0; sb < 4; ++sb)
+                        if ((mask >> sb) & 1) {
+                            a0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[sb], W[sb][0], a0, 0, 0, 0);
+                            a1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[sb], W[sb][1], a1, 0, 0, 0);
+                            a2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[sb], W[sb][2], a2, 0, 0, 0);
+                            a3 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[sb], W[sb][3], a3, 0, 0, 0);
+                        }
+                    const int slots = __builtin_amdgcn_readlane(tr.y, ti);
+                    // the next tile's operands (past the last: zeros), on their way during this one's flush
+                    ++ti;
+                    mask = __builtin_amdgcn_readlane(tr.x, ti & 15) & (ti < nt ? 15 : 0);
+                    load_tile();
+                    // lane: class zq of the tile, lead column lane & 15, coefficient in the register
+                    double v[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        v[q] = __builtin_fma((double)(a2[q] + 256 * a3[q]), 65536.0, (double)(a0[q] + 256 * a1[q]));
+                    const double g = __builtin_fma(v[0], cz, __builtin_fma(v[1], cy, __builtin_fma(v[2], cx, v[3] * sc)));
+                    s_acc[w][((unsigned)slots >> (8 * zq)) & 255u][lane & 15] += g;
+                    if (ti >= nt) break;
+                }
+                if (!hot || !__any(np > pass + 1)) break;
+                sc *= 0x1p-30;
+            }
         }
-        double* os = sums + (R.c_off + H.n_chunks + (int64_t)k * CW + i) * 3 * LP;
-        os[ld] = sg;
-        os[LP + ld] = pp * sg;
-        os[2 * LP + ld] = qq * sg;
+        __syncthreads();
+        double* out = gsum + (sg.goff + (int64_t)rg * n_lines + reg.z) * 16;
+        for (int i = t; i < reg.w * 16; i += 64 * CB_WAVES) {
+            double v = 0.0;
+#pragma unroll
+            for (int q = 0; q < CB_WAVES; ++q) v += (&s_acc[q][0][0])[i];
+            out[i] = v;
+        }
+        __syncthreads();
     }
 }
 
-// csums[(cls_off + k)*3*LP + v]: the sums of class k (k0 sum G, sum G P',
-// sum G Q' per lead, k0 the class's layer's resting value), its window's
-// pieces added in order.
+// csums[(cls_off + k)*3*LP + v]: the sums of class k for each row (request,
+// lead) of a launch's 16-lead rows: k0 sum G, P' sum G, Q' sum G, with the
+// sum over the class's regions in order, k0 the class's layer's resting value
+// and P' = k2(1-k3) e^{(k4+k5)(a - t0)}, Q' = k2 k3 e^{k5 (a - t0)}.  The
+// thread of a request's last lead also clears the unused lead slots.
 template <int LP>
-__global__ void class_sums_kernel(const HeartDev* __restrict__ hearts, const ReqDev* __restrict__ reqs, int B,
-                                  const int64_t* __restrict__ cs_start, const double* __restrict__ layer_k,
-                                  const double* __restrict__ sums, double* __restrict__ csums)
+__global__ __launch_bounds__(256) void class_sums_kernel(
+    const HeartDev* __restrict__ hearts, const ReqDev* __restrict__ reqs, const ClassSeg* __restrict__ segs,
+    const int* __restrict__ rgseg, const int* __restrict__ rowtab, int rg0, const double* __restrict__ layer_k,
+    const double* __restrict__ gsum, double* __restrict__ csums)
 {
-    // grid rows over the requests (the request is block-uniform), columns
-    // over a request's (class, column) items
-    for (int r = blockIdx.y; r < B; r += gridDim.y) {
-        const int64_t c0 = cs_start[r];
-        const int64_t n = (cs_start[r + 1] - c0) * 3 * LP;
-        if (n == 0) continue;
-        const ReqDev& R = reqs[r];
-        const HeartDev& H = hearts[R.heart];
-        for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < n;
-             idx += (int64_t)gridDim.x * blockDim.x) {
-            const int k = (int)(idx / (3 * LP));
-            const int v = (int)(idx - (int64_t)k * (3 * LP));
-            const int wi = k / CLASS_WINDOW, i = k - wi * CLASS_WINDOW;
-            double s = 0.0;
-            for (int p = H.cwin[wi]; p < H.cwin[wi + 1]; ++p)
-                s += sums[(R.c_off + H.n_chunks + (int64_t)p * CLASS_WINDOW + i) * 3 * LP + v];
-            if (v < LP) s *= layer_k[R.k_off + 9 * (H.classes[k].x - 1)];
-            csums[(c0 + k) * 3 * LP + v] = s;
-        }
-    }
+    const int rg = rg0 + blockIdx.y, t = threadIdx.x;
+    const ClassSeg sg = segs[rgseg[rg]];
+    const HeartDev& H = hearts[sg.heart];
+    const int k = blockIdx.x * 16 + (t >> 4);
+    const int row = rowtab[16 * rg + (t & 15)];
+    if (k >= H.n_classes || row < 0) return;
+    const double* g = gsum + (sg.goff + (int64_t)(rg - sg.rg0) * H.n_lines) * 16 + (t & 15);
+    double s = 0.0;
+    const int q1 = H.cs_off[k + 1];
+#pragma unroll 4
+    for (int q = H.cs_off[k]; q < q1; ++q) s += g[(int64_t)16 * H.cs_line[q]];
+    const ReqDev& R = reqs[row >> 5];
+    const int i = row & 31, l = H.classes[k].x;
+    const double* kk = layer_k + R.k_off + 9 * (l - 1);
+    const double da = H.class_a[k] - H.layer_t0[l];
+    double* o = csums + (R.cls_off + k) * 3 * LP;
+    o[i] = s * kk[0];
+    o[LP + i] = kk[2] * (1.0 - kk[3]) * exp((kk[4] + kk[5]) * da) * s;
+    o[2 * LP + i] = kk[2] * kk[3] * exp(kk[5] * da) * s;
+    if (i == R.L - 1)
+        for (int z = R.L; z < LP; ++z) o[z] = o[LP + z] = o[2 * LP + z] = 0.0;
 }
 
 // ecg[r][i][t] += sum over the heart's activation classes of
@@ -1646,35 +1780,23 @@ hipError_t launch_ecg_chunk(const GroupArgs& a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_class_windows(const GroupArgs& a, hipStream_t s)
+hipError_t launch_class_boxes(const GroupArgs& a, const ClassLaunch& c, hipStream_t s)
 {
-    if (a.n_cc == 0) return hipSuccess;
-    if (a.n_cc > 0x7fffffffLL) return hipErrorInvalidValue;
-    switch (a.LP) {
-#define EKG_CWIN(LPV)                                                                                        \
-    case LPV:                                                                                                \
-        hipLaunchKernelGGL(ecg_class_window_kernel<LPV>, dim3((unsigned)a.n_cc), dim3(CC_THREADS), 0, s, a.hearts, \
-                           a.reqs, a.cc_runs, a.cc_rstart, a.n_runs, a.lead_pos, a.layer_k, a.sums);       \
-        break;
-        EKG_CWIN(4)
-        EKG_CWIN(8)
-        EKG_CWIN(12)
-        EKG_CWIN(16)
-#undef EKG_CWIN
-    default: return hipErrorInvalidValue;
-    }
+    if (c.blocks < 1 || c.blocks > 0x7fffffffLL || c.n_segs < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(ecg_class_box_kernel, dim3((unsigned)c.blocks), dim3(64 * CB_WAVES), 0, s, a.hearts,
+                       a.segs + c.seg0, c.n_segs, a.rowpos, a.lead_pos, a.gsum);
     return hipGetLastError();
 }
 
-hipError_t launch_class_sums(const GroupArgs& a, hipStream_t s)
+hipError_t launch_class_sums(const GroupArgs& a, const ClassLaunch& c, hipStream_t s)
 {
-    if (a.n_cs == 0) return hipSuccess;
+    if (c.n_rg < 1 || c.n_rg > 65535 || a.cs_max < 1) return hipErrorInvalidValue;
     switch (a.LP) {
-#define EKG_CSUMS(LPV)                                                                                  \
-    case LPV:                                                                                           \
-        hipLaunchKernelGGL(class_sums_kernel<LPV>,                                                     \
-                           dim3(grid_for((int64_t)a.cs_max * 3 * LPV, 256), std::min(a.B, 65535)), dim3(256), \
-                           0, s, a.hearts, a.reqs, a.B, a.cs_start, a.layer_k, a.sums, a.csums);         \
+#define EKG_CSUMS(LPV)                                                                                       \
+    case LPV:                                                                                                \
+        hipLaunchKernelGGL(class_sums_kernel<LPV>, dim3((unsigned)((a.cs_max + 15) / 16), (unsigned)c.n_rg), \
+                           dim3(256), 0, s, a.hearts, a.reqs, a.segs, a.rgseg, a.rowtab, c.rg0, a.layer_k,   \
+                           a.gsum, a.csums);                                                                 \
         break;
         EKG_CSUMS(4)
         EKG_CSUMS(8)
@@ -1726,7 +1848,6 @@ static void prime_lp(hipFuncAttributes& at)
     prime_nh<LP, 1>(at);
     prime_nh<LP, 2>(at);
     prime_nh<LP, 3>(at);
-    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_window_kernel<LP>);
     (void)hipFuncGetAttributes(&at, (const void*)class_sums_kernel<LP>);
     (void)hipFuncGetAttributes(&at, (const void*)layer_prefix_kernel<LP>);
     (void)hipFuncGetAttributes(&at, (const void*)ecg_reduce_kernel<LP>);
@@ -1737,6 +1858,7 @@ void prime_kernels()
 {
     hipFuncAttributes at;
     (void)hipFuncGetAttributes(&at, (const void*)ap_tables_kernel);
+    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel);
     prime_lp<4>(at);
     prime_lp<8>(at);
     prime_lp<12>(at);

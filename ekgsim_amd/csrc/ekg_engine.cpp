@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <numeric>
+#include <type_traits>
 #include <unordered_map>
 
 namespace ekg {
@@ -255,9 +256,21 @@ constexpr int DEFAULT_CLASS_MIN = 64;
 // Largest class chunk (voxels): a class is kept as a run of class chunks
 // (layout bookkeeping; the class-window kernel takes whole classes).
 constexpr int64_t CLASS_CHUNK = 4096;
-// Classes per class window and groups of 16 entries per piece (see ensure_cells).
-constexpr int CLASS_WINDOW = ekgk::CLASS_WINDOW;
-constexpr int CLASS_PIECE = ekgk::CLASS_PIECE;
+// Windows of six classes and pieces of 1024 groups of 16 window entries: the
+// units in which layout_info states a layout's size, and the fixed workspace
+// its share of class sums.
+constexpr int CLASS_WINDOW = 6;
+constexpr int64_t CLASS_PIECE = 1024;
+// Class boxes: 4 x 8 x 8 cells (z, y, x) in four sub-bricks of 4^3; a region
+// takes about 1/64 of a heart's boxes, at least 4 (one per wave of its block)
+// and at most 64.
+constexpr int BOX_Z = 4, BOX_Y = 8, BOX_X = 8;
+constexpr int CB_SLOTS = ekgk::CB_SLOTS;
+constexpr size_t BOX_CLASSES = 64;  // classes of one listing of a box (16 tiles)
+// Most bytes of class sums per launch; a larger group runs its rows in
+// several launches.
+constexpr int64_t GSUM_BYTES = (int64_t)256 << 20;
+constexpr int64_t LINE_BYTES = 16 * 8;
 
 namespace {
 // Chunk size: DEFAULT_CHUNK voxels unless the heart is tuned.  Chunks are
@@ -558,35 +571,22 @@ void ensure_layout(Heart& h, bool mfma)
 // this sum; a cell w has grid coordinates + 1 (the reference's voxel centre)
 // c(w), D(w) and its moment K(w) = -D(w) . c(w), all integers.
 //
-// A cell borders several classes (4 to 5 on average on a heart with delays of
-// 1 to 3 ms per voxel), and its lead weight s(w) = |p - c(w)|^-3 is the same
-// for all of them.  So the classes are taken CLASS_WINDOW at a time (in layer
-// and time order): an entry is a cell with a non-zero D for at least one
-// class of the window, and the class-window kernel evaluates each entry's
-// weight once per lead and request and adds it, times the entry's D and K for
-// class i of the window, to that class's sums.  Entries are sorted by their
-// class mask and cut into groups of 16; a group lists, for every class of its
-// mask (the union of its entries'), the 64 lanes' coefficients, and the
-// kernel runs one matrix product per class of the mask.
-//
-// Each of the 64 lanes feeds the matrix products fixed operands of its group
-// (lane = 16 kq + 4 b + rc, entry index within the group el = 4 b + kq,
-// ea = 4 b + rc):
-//   av = coordinate kq of entry ea (kq = 3: 1),
-//   cc = |c|^2 of entry el,
-//   bv = coefficient rc of entry el for class i: D_0, D_1, D_2 (rc < 3) or K.
-// They are stored lane-major, as FP32 (every value is an integer below 2^24,
-// exact): group q occupies rows crow[q].x, ... of 64 floats in cgrp: av, cc,
-// then bv for each class of its mask in order; crow[q].y is the mask.  A
-// group's missing entries (past the window's last) repeat its first entry
-// with coefficients 0, so their weights are finite and add nothing.
-//
-// For parallelism a window's groups are cut into the fewest pieces of at
-// most CLASS_PIECE groups, of equal size up to one group (so that no block
-// is left with a short remainder), one block per (piece, request); each writes its sums
-// for all CLASS_WINDOW classes, and class_sums_kernel adds a class's pieces
-// in order.  The cut depends on the heart only, so a request's ECG does not
-// depend on the batch it runs in.
+// The class-box kernel evaluates a cell's weight once and adds it to every
+// class with a non-zero D there.  Layout, per neighbourhood:
+//  * The cells are taken in boxes of 4 x 8 x 8 (aligned in the grid, in Morton
+//    order), each in four sub-bricks of 4^3 cells.
+//  * A box's classes, in order, are cut into tiles of 4; for each sub-brick with
+//    cells of a tile's classes there is one coefficient block, the int8 operand of
+//    v_mfma_i32_16x16x64_i8: lane 16 z + 4 class + coefficient, byte 4 y + x holds
+//    D_z, D_y, D_x or K = -D . (c - c0) of the cell, c0 the box's first cell
+//    (|D| <= 9 and, for any set of neighbours, |K| <= 93).  The kernel
+//    feeds each byte of a weight less 128, so a tile's accumulators start at 128
+//    times the sum of their coefficients.
+//  * Consecutive boxes form regions with at most CB_SLOTS classes, whose sums
+//    a block keeps in LDS; a box with more classes is listed again with the rest.
+//    Each (region, class) has a line of sums, listed per class in order.
+// The cut depends on the heart only, so a request's ECG does not depend on
+// the batch it runs in.
 void ensure_cells(Heart& h, int nhood)
 {
     EcgLayout& L = h.layout;
@@ -594,28 +594,22 @@ void ensure_cells(Heart& h, int nhood)
     if (L.cells_built[nhood]) return;
     int8_t dif[26][3];
     const int nd = nhood_offsets(nhood, dif);
-    // cell -> entry of the current window (-1: none), reset after each
-    // window: a dense array over the grid, or a hash map for grids above
-    // 2^27 cells (the array would exceed 512 MB)
+    // cell -> index among the current class's cells (-1: none): a dense array
+    // over the grid, or a hash map for grids above 2^27 cells (the array would
+    // exceed 512 MB)
     const bool dense = h.nvox <= ((int64_t)1 << 27);
-    std::vector<int> slot(dense ? (size_t)h.nvox : 0, -1);
-    std::unordered_map<int64_t, int> slot_map;
     std::vector<int64_t> touched;   // cells of the current class, first-touch order
     std::vector<int> acc;           // D per touched cell, three ints
-    std::vector<int> tslot(dense ? (size_t)h.nvox : 0, -1);  // cell -> touched index of the current class
+    std::vector<int> tslot(dense && L.n_classes > 0 ? (size_t)h.nvox : 0, -1);
     std::unordered_map<int64_t, int> tslot_map;
-    struct Entry {
-        int c[3];
-        int mask;
-        int first;  // first touch (order within a mask)
-        int coef[CLASS_WINDOW][4];
+    struct Rec {  // a cell with a non-zero D for a class
+        int box, cls;
+        uint8_t cell;  // 64 sub-brick + 16 z + 4 y + x within the box
+        int8_t d[3];
     };
-    std::vector<Entry> ent;
-    std::vector<float> grp;          // rows of 64 floats
-    std::vector<int2> crow;          // per group: first row, class mask
-    std::vector<int4> pieces;        // {window, first group, end group, 0}
-    std::vector<int> wpiece(1, 0);   // pieces of window w: [wpiece[w], wpiece[w+1])
-    int64_t n_cells = 0, n_entries = 0;
+    std::vector<Rec> recs;
+    const int nb1 = (h.n1 + BOX_Y - 1) / BOX_Y, nb2 = (h.n2 + BOX_X - 1) / BOX_X;
+    std::vector<int64_t> box_begin((size_t)((h.n0 + BOX_Z - 1) / BOX_Z) * nb1 * nb2 + 1, 0);
     auto bit = [](int d0, int d1, int d2) { return (d0 + 1) * 9 + (d1 + 1) * 3 + (d2 + 1); };
     auto add = [&](int z, int y, int x, int d0, int d1, int d2) {
         const int64_t gi = ((int64_t)z * h.n1 + y) * h.n2 + x;
@@ -634,138 +628,230 @@ void ensure_cells(Heart& h, int nhood)
         acc[3 * sl + 1] += d1;
         acc[3 * sl + 2] += d2;
     };
-    const int n_win = (L.n_classes + CLASS_WINDOW - 1) / CLASS_WINDOW;
-    for (int w = 0; w < n_win; ++w) {
-        ent.clear();
-        const int k0 = w * CLASS_WINDOW, k1 = std::min(L.n_classes, k0 + CLASS_WINDOW);
-        for (int k = k0; k < k1; ++k) {
-            // the class's voxels: those of its class chunks, which are consecutive
-            const int4 cl = L.h_classes[k];
-            const int v_begin = L.h_cchunks[cl.y].y, v_end = L.h_cchunks[cl.z - 1].z;
-            touched.clear();
-            acc.clear();
-            for (int v = v_begin; v < v_end; ++v) {
-                const uint2 g = L.h_geo[v];
-                const int z = (int)(g.x & 1023u), y = (int)((g.x >> 10) & 1023u), x = (int)(g.x >> 20);
-                int s0 = 0, s1 = 0, s2 = 0;
-                for (int q = 0; q < nd; ++q) {
-                    if (!((g.y >> bit(dif[q][0], dif[q][1], dif[q][2])) & 1u)) continue;
-                    add(z + dif[q][0], y + dif[q][1], x + dif[q][2], dif[q][0], dif[q][1], dif[q][2]);
-                    s0 += dif[q][0];
-                    s1 += dif[q][1];
-                    s2 += dif[q][2];
-                }
-                add(z, y, x, s0, s1, s2);
+    for (int k = 0; k < L.n_classes; ++k) {
+        // the class's voxels: those of its class chunks, which are consecutive
+        const int4 cl = L.h_classes[k];
+        const int v_begin = L.h_cchunks[cl.y].y, v_end = L.h_cchunks[cl.z - 1].z;
+        touched.clear();
+        acc.clear();
+        for (int v = v_begin; v < v_end; ++v) {
+            const uint2 g = L.h_geo[v];
+            const int z = (int)(g.x & 1023u), y = (int)((g.x >> 10) & 1023u), x = (int)(g.x >> 20);
+            int s0 = 0, s1 = 0, s2 = 0;
+            for (int q = 0; q < nd; ++q) {
+                if (!((g.y >> bit(dif[q][0], dif[q][1], dif[q][2])) & 1u)) continue;
+                add(z + dif[q][0], y + dif[q][1], x + dif[q][2], dif[q][0], dif[q][1], dif[q][2]);
+                s0 += dif[q][0];
+                s1 += dif[q][1];
+                s2 += dif[q][2];
             }
-            tslot_map.clear();
-            for (size_t t = 0; t < touched.size(); ++t) {
-                const int64_t gi = touched[t];
-                if (dense) tslot[gi] = -1;
-                const int D0 = acc[3 * t], D1 = acc[3 * t + 1], D2 = acc[3 * t + 2];
-                if (!(D0 || D1 || D2)) continue;
-                if (std::abs(D0) > 127 || std::abs(D1) > 127 || std::abs(D2) > 127)
-                    fail(EKG_EINVAL, "dipole vector out of range");
-                ++n_cells;
-                int e;
-                if (dense) {
-                    e = slot[gi];
-                    if (e < 0) e = slot[gi] = (int)ent.size();
-                } else {
-                    e = slot_map.emplace(gi, (int)ent.size()).first->second;
-                }
-                if (e == (int)ent.size()) {
-                    const int x = (int)(gi % h.n2), y = (int)((gi / h.n2) % h.n1),
-                              z = (int)(gi / ((int64_t)h.n2 * h.n1));
-                    Entry en{};
-                    en.c[0] = z + 1;
-                    en.c[1] = y + 1;
-                    en.c[2] = x + 1;
-                    en.first = e;
-                    ent.push_back(en);
-                }
-                Entry& en = ent[e];
-                const int i = k - k0;
-                en.mask |= 1 << i;
-                en.coef[i][0] = D0;
-                en.coef[i][1] = D1;
-                en.coef[i][2] = D2;
-                en.coef[i][3] = -(D0 * en.c[0] + D1 * en.c[1] + D2 * en.c[2]);
-            }
+            add(z, y, x, s0, s1, s2);
         }
-        // reset the cell -> entry map for the next window
-        if (dense)
-            for (const Entry& en : ent)
-                slot[((int64_t)(en.c[0] - 1) * h.n1 + (en.c[1] - 1)) * h.n2 + (en.c[2] - 1)] = -1;
-        else
-            slot_map.clear();
-        // entries by (lowest class, mask, first touch): groups of like masks
-        std::sort(ent.begin(), ent.end(), [](const Entry& x, const Entry& y) {
-            const int fx = __builtin_ctz((unsigned)x.mask), fy = __builtin_ctz((unsigned)y.mask);
-            if (fx != fy) return fx < fy;
-            if (x.mask != y.mask) return x.mask < y.mask;
-            return x.first < y.first;
-        });
-        const int g_begin = (int)crow.size();
-        const size_t ne = ent.size();
-        n_entries += (int64_t)ne;
-        for (size_t q0 = 0; q0 < ne; q0 += 16) {
-            int mask = 0;
-            for (size_t e = q0; e < std::min(ne, q0 + 16); ++e) mask |= ent[e].mask;
-            const int nrow = 2 + __builtin_popcount((unsigned)mask);
-            if (grp.size() / 64 + nrow > 0x7fffffffu) fail(EKG_EINVAL, "too many class cells");
-            crow.push_back(make_int2((int)(grp.size() / 64), mask));
-            const size_t base = grp.size();
-            grp.resize(base + (size_t)64 * nrow);
-            float* av = grp.data() + base;
-            float* sq = av + 64;
-            for (int lane = 0; lane < 64; ++lane) {
-                const int kq = lane >> 4, b = (lane >> 2) & 3, rc = lane & 3;
-                const size_t el = q0 + 4 * b + kq, ea = q0 + 4 * b + rc;
-                const Entry& A = ent[ea < ne ? ea : q0];
-                const bool ok = el < ne;
-                const Entry& C = ent[ok ? el : q0];
-                av[lane] = kq < 3 ? (float)A.c[kq] : 1.0f;
-                sq[lane] = (float)(C.c[0] * C.c[0] + C.c[1] * C.c[1] + C.c[2] * C.c[2]);
-                int r = 2;
-                for (int i = 0; i < CLASS_WINDOW; ++i) {
-                    if (!((mask >> i) & 1)) continue;
-                    av[64 * r + lane] = ok ? (float)C.coef[i][rc] : 0.0f;
-                    ++r;
-                }
-            }
+        tslot_map.clear();
+        for (size_t t = 0; t < touched.size(); ++t) {
+            const int64_t gi = touched[t];
+            if (dense) tslot[gi] = -1;
+            const int D0 = acc[3 * t], D1 = acc[3 * t + 1], D2 = acc[3 * t + 2];
+            if (!(D0 || D1 || D2)) continue;
+            if (std::abs(D0) > 9 || std::abs(D1) > 9 || std::abs(D2) > 9) fail(EKG_EINVAL, "dipole vector out of range");
+            const int x = (int)(gi % h.n2), y = (int)((gi / h.n2) % h.n1), z = (int)(gi / ((int64_t)h.n2 * h.n1));
+            const int box = ((z / BOX_Z) * nb1 + y / BOX_Y) * nb2 + x / BOX_X;
+            const int sub = 2 * ((y / 4) & 1) + ((x / 4) & 1);
+            recs.push_back(Rec{box, k, (uint8_t)(64 * sub + 16 * (z & 3) + 4 * (y & 3) + (x & 3)),
+                               {(int8_t)D0, (int8_t)D1, (int8_t)D2}});
+            ++box_begin[box + 1];
         }
-        const int g_end = (int)crow.size();
-        // at least one piece per window, so every class has sums (0 without entries)
-        const int n_pc = std::max(1, (g_end - g_begin + CLASS_PIECE - 1) / CLASS_PIECE);
-        const int pc_size = std::max(1, (g_end - g_begin + n_pc - 1) / n_pc);
-        int g = g_begin;
-        do {
-            const int ge = std::min(g_end, g + pc_size);
-            pieces.push_back(int4{w, g, ge, 0});
-            g = ge;
-        } while (g < g_end);
-        wpiece.push_back((int)pieces.size());
     }
-    L.n_ccells[nhood] = n_cells;
-    L.n_centries[nhood] = n_entries;
-    L.n_cgroups[nhood] = (int64_t)crow.size();
-    L.n_cpieces[nhood] = (int)pieces.size();
-    if (grp.empty()) grp.assign(64, 0.0f);
-    if (crow.empty()) crow.push_back(make_int2(0, 0));
-    if (pieces.empty()) pieces.push_back(int4{0, 0, 0, 0});
+    // records by box, each box's by class (counting sort, stable)
+    std::vector<std::pair<uint64_t, int>> order;  // used boxes in Morton order
+    for (size_t q = 0; q + 1 < box_begin.size(); ++q) {
+        if (box_begin[q + 1]) {
+            const uint32_t bx = (uint32_t)(q % nb2), by = (uint32_t)((q / nb2) % nb1), bz = (uint32_t)(q / nb2 / nb1);
+            uint64_t code = 0;
+            for (int i = 0; i < 12; ++i)
+                code |= (uint64_t)((bx >> i) & 1) << (3 * i + 1) | (uint64_t)((by >> i) & 1) << (3 * i + 2) |
+                        (uint64_t)((bz >> (i + 1)) & 1) << (3 * i + 3);
+            order.push_back({code | (bz & 1), (int)q});
+        }
+        box_begin[q + 1] += box_begin[q];
+    }
+    std::sort(order.begin(), order.end());
+    std::vector<Rec> sorted(recs.size());
+    {
+        std::vector<int64_t> at(box_begin.begin(), box_begin.end() - 1);
+        for (const Rec& r : recs) sorted[at[r.box]++] = r;
+        std::vector<Rec>().swap(recs);
+    }
+    int64_t n_entries = 0;
+    std::vector<int64_t> win_entries((L.n_classes + CLASS_WINDOW - 1) / CLASS_WINDOW, 0);
+    std::vector<int4> regions, ext;           // ext: a region's first and last cells + 1 per axis
+    int n_box = 0;                            // listed boxes
+    std::vector<int4> pkt;                    // 64 per listed box: its tiles' records, its own
+    std::vector<int> init;                    // 256 per listed box: 16 per tile
+    std::vector<int8_t> coef;                 // 1024 per block
+    std::vector<uint64_t> mask;               // 4 per listed box
+    std::vector<std::pair<int, int>> lines;   // (class, line)
+    std::vector<int> slot_of(L.n_classes, -1), slot_cls;  // slots of the current region
+    const int target = (int)std::min<size_t>(64, std::max<size_t>(4, (order.size() / 64 + 3) / 4 * 4));
+    std::vector<int> cost;  // per listed box of the current region
+    auto close = [&]() {
+        int4& r = regions.back();
+        r.y = n_box;
+        // The block's wave w takes boxes w, w + 4, ...: order them so that
+        // the waves' work is about equal (largest first, each to the wave with
+        // least so far that still has a place).
+        const int n = r.y - r.x, nw = ekgk::CB_WAVES;
+        std::vector<int> by(n), at(n);
+        std::iota(by.begin(), by.end(), 0);
+        std::stable_sort(by.begin(), by.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+        std::vector<int64_t> load(nw, 0);
+        std::vector<int> cnt(nw, 0);
+        for (int i : by) {
+            int w = -1;
+            for (int q = 0; q < nw; ++q)
+                if (cnt[q] * nw + q < n && (w < 0 || load[q] < load[w])) w = q;
+            at[i] = cnt[w]++ * nw + w;
+            load[w] += cost[i];
+        }
+        cost.clear();
+        auto reorder = [&](auto& v, size_t per) {
+            std::remove_reference_t<decltype(v)> tmp(v.begin() + (std::ptrdiff_t)(per * r.x), v.end());
+            for (int i = 0; i < n; ++i)
+                std::copy_n(tmp.begin() + (std::ptrdiff_t)(per * i), per, v.begin() + (std::ptrdiff_t)(per * (r.x + at[i])));
+        };
+        reorder(pkt, 64);
+        reorder(init, 256);
+        reorder(mask, 4);
+        r.w = (int)slot_cls.size();
+        for (size_t i = 0; i < slot_cls.size(); ++i) {
+            lines.push_back({slot_cls[i], r.z + (int)i});
+            slot_of[slot_cls[i]] = -1;
+        }
+        slot_cls.clear();
+    };
+    std::vector<int> cls;   // the box's classes
+    for (const auto& ob : order) {
+        const Rec* r0 = sorted.data() + box_begin[ob.second];
+        const Rec* r1 = sorted.data() + box_begin[ob.second + 1];
+        const int bx = ob.second % nb2, by = (ob.second / nb2) % nb1, bz = ob.second / nb2 / nb1;
+        int last_win[256];
+        std::fill(last_win, last_win + 256, -1);
+        cls.clear();
+        for (const Rec* r = r0; r < r1; ++r) {
+            if (cls.empty() || cls.back() != r->cls) cls.push_back(r->cls);
+            const int w = r->cls / CLASS_WINDOW;
+            if (last_win[r->cell] != w) {
+                last_win[r->cell] = w;
+                ++win_entries[w];
+                ++n_entries;
+            }
+        }
+        for (size_t c0 = 0; c0 < cls.size(); c0 += BOX_CLASSES) {
+            const size_t c1 = std::min(cls.size(), c0 + BOX_CLASSES);
+            size_t fresh = 0;
+            for (size_t c = c0; c < c1; ++c) fresh += slot_of[cls[c]] < 0;
+            if (regions.empty() || slot_cls.size() + fresh > (size_t)CB_SLOTS ||
+                n_box - regions.back().x >= target) {
+                if (!regions.empty()) close();
+                regions.push_back(int4{n_box, 0, (int)lines.size(), 0});
+                ext.push_back(int4{0xffff, 0xffff, 0xffff, 0});
+            }
+            for (size_t c = c0; c < c1; ++c)
+                if (slot_of[cls[c]] < 0) {
+                    slot_of[cls[c]] = (int)slot_cls.size();
+                    slot_cls.push_back(cls[c]);
+                }
+            const size_t blk0 = coef.size() / 1024;
+            const int n_tile = (int)((c1 - c0 + 3) / 4);
+            const size_t pk = 64 * (size_t)n_box;
+            pkt.resize(pk + 64, int4{0, 0, 0, 0});
+            init.resize(256 * (size_t)n_box + 256, 0);
+            const Rec* r = r0;
+            while (r < r1 && r->cls < cls[c0]) ++r;
+            int used = 0;
+            uint64_t bm[4] = {0, 0, 0, 0};
+            for (int t = 0; t < n_tile; ++t) {
+                const size_t q0 = c0 + 4 * t, q1 = std::min(c1, q0 + 4);
+                unsigned slots = 0;
+                for (size_t q = q0; q < q0 + 4; ++q)
+                    slots |= (unsigned)(q < q1 ? slot_of[cls[q]] : CB_SLOTS) << (8 * (q - q0));
+                const Rec* rt = r;
+                int subs = 0;
+                for (; r < r1 && r->cls <= cls[q1 - 1]; ++r) subs |= 1 << (r->cell >> 6);
+                if (coef.size() / 1024 > 0x7ffffff0u) fail(EKG_EINVAL, "too many class cells");
+                const size_t base = coef.size(), ib = 256 * (size_t)n_box + 16 * t;
+                pkt[pk + t] = int4{subs, (int)slots, (int)(base / 1024), 0};
+                coef.resize(base + 1024 * (size_t)__builtin_popcount((unsigned)subs), 0);
+                size_t q = q0;
+                for (; rt < r; ++rt) {
+                    while (cls[q] != rt->cls) ++q;
+                    const int sub = rt->cell >> 6, z = (rt->cell >> 4) & 3, y = (rt->cell >> 2) & 3, x = rt->cell & 3;
+                    const int dz = z, dy = y + 4 * (sub >> 1), dx = x + 4 * (sub & 1);
+                    const int K = -(rt->d[0] * dz + rt->d[1] * dy + rt->d[2] * dx);
+                    if (K < -127 || K > 127) fail(EKG_EINVAL, "dipole moment out of range");
+                    const int row = 4 * (int)(q - q0);
+                    const int co[4] = {rt->d[0], rt->d[1], rt->d[2], K};
+                    const size_t blk = base + 1024 * (size_t)__builtin_popcount((unsigned)(subs & ((1 << sub) - 1)));
+                    bm[sub] |= (uint64_t)1 << (rt->cell & 63);
+                    used |= 1 << (4 * sub + y);
+                    for (int i = 0; i < 4; ++i) {
+                        coef[blk + 16 * (16 * z + row + i) + 4 * y + x] = (int8_t)co[i];
+                        init[ib + row + i] += 128 * co[i];
+                    }
+                }
+            }
+            const int o[3] = {bz * BOX_Z + 1, by * BOX_Y + 1, bx * BOX_X + 1};
+            pkt[pk + 16] = int4{n_tile, used, 0, 0};
+            pkt[pk + 17] = int4{o[0], o[1], o[2], 0};
+            // cycles of a box, roughly: 34 a weight of 64 lanes, 64 a block's
+            // four products, 180 a tile's flush
+            cost.push_back(500 + 136 * __builtin_popcount((unsigned)used) +
+                           64 * (int)(coef.size() / 1024 - blk0) + 180 * n_tile);
+            ++n_box;
+            const int len[3] = {BOX_Z, BOX_Y, BOX_X};
+            int* e = &ext.back().x;
+            for (int i = 0; i < 3; ++i)
+                e[i] = std::min(e[i] & 0xffff, o[i]) | std::max(e[i] >> 16, o[i] + len[i] - 1) << 16;
+            mask.insert(mask.end(), bm, bm + 4);
+        }
+    }
+    if (!regions.empty()) close();
+    int64_t n_pieces = 0;
+    for (int64_t ne : win_entries) {
+        const int64_t groups = (ne + 15) / 16, pc = std::max<int64_t>(1, (groups + CLASS_PIECE - 1) / CLASS_PIECE);
+        const int64_t size = std::max<int64_t>(1, (groups + pc - 1) / pc);
+        n_pieces += std::max<int64_t>(1, (groups + size - 1) / size);
+    }
+    // lines per class, in region order
+    std::vector<int> cs_off(L.n_classes + 1, 0), cs_line(lines.size());
+    for (const auto& l : lines) ++cs_off[l.first + 1];
+    for (int k = 0; k < L.n_classes; ++k) cs_off[k + 1] += cs_off[k];
+    {
+        std::vector<int> at(cs_off.begin(), cs_off.end() - 1);
+        for (const auto& l : lines) cs_line[at[l.first]++] = l.second;
+    }
     h.ctx->bind();
-    L.cgrp[nhood].reserve(grp.size() * sizeof(float));
-    L.crow[nhood].reserve(crow.size() * sizeof(int2));
-    L.cpieces[nhood].reserve(pieces.size() * sizeof(int4));
-    L.cwin[nhood].reserve(wpiece.size() * sizeof(int));
-    hip_check(hipMemcpy(L.cgrp[nhood].p, grp.data(), grp.size() * sizeof(float), hipMemcpyHostToDevice),
-              "upload class cell groups");
-    hip_check(hipMemcpy(L.crow[nhood].p, crow.data(), crow.size() * sizeof(int2), hipMemcpyHostToDevice),
-              "upload class cell group rows");
-    hip_check(hipMemcpy(L.cpieces[nhood].p, pieces.data(), pieces.size() * sizeof(int4), hipMemcpyHostToDevice),
-              "upload class window pieces");
-    hip_check(hipMemcpy(L.cwin[nhood].p, wpiece.data(), wpiece.size() * sizeof(int), hipMemcpyHostToDevice),
-              "upload class window piece offsets");
+    auto upload = [&](DevBuf& b, const void* p, size_t n, const char* what) {
+        b.reserve(std::max<size_t>(n, 16));
+        if (n) hip_check(hipMemcpy(b.p, p, n, hipMemcpyHostToDevice), what);
+    };
+    std::vector<int4> reg2;
+    for (size_t i = 0; i < regions.size(); ++i) {
+        reg2.push_back(regions[i]);
+        reg2.push_back(ext[i]);
+    }
+    upload(L.cregion[nhood], reg2.data(), reg2.size() * sizeof(int4), "upload class regions");
+    upload(L.cbox[nhood], pkt.data(), pkt.size() * sizeof(int4), "upload class boxes");
+    upload(L.cinit[nhood], init.data(), init.size() * sizeof(int), "upload class tile starts");
+    upload(L.ccoef[nhood], coef.data(), coef.size(), "upload class coefficients");
+    upload(L.cmask[nhood], mask.data(), mask.size() * sizeof(uint64_t), "upload class cell masks");
+    upload(L.cs_off[nhood], cs_off.data(), cs_off.size() * sizeof(int), "upload class lines");
+    upload(L.cs_line[nhood], cs_line.data(), cs_line.size() * sizeof(int), "upload class lines");
+    L.n_ccells[nhood] = (int64_t)sorted.size();
+    L.n_centries[nhood] = n_entries;
+    L.n_cpieces[nhood] = (int)n_pieces;
+    L.n_lines[nhood] = (int)lines.size();
+    L.n_regions[nhood] = (int)regions.size();
     L.cells_built[nhood] = true;
 }
 
@@ -773,18 +859,24 @@ namespace {
 
 // Per-request sizes of a group's packed arrays.
 struct ReqSizes {
-    int64_t rows, chunks, mixed, cchunks, bricks, classes;
+    int64_t rows, chunks, bricks, classes;
 };
 
 ReqSizes req_sizes(const ReqSpec& r, bool mfma)
 {
     const EcgLayout& L = r.h->layout;
-    // the chunk kernel (matrix-core path) keeps G rows on chip: no records;
-    // per-chunk sums for the chunks outside classes and per (class-window
-    // piece, class of the window), partial rows for chunks outside classes
-    const int64_t pieces = mfma ? L.n_cpieces[r.nhood] : 0;
-    return ReqSizes{mfma ? 0 : L.V + ekgk::MFMA_PAD, (int64_t)L.n_chunks + pieces * CLASS_WINDOW, L.n_chunks,
-                    pieces, L.n_bricks, L.n_classes};
+    // the chunk kernel (matrix-core path) keeps G rows on chip: no records
+    return ReqSizes{mfma ? 0 : L.V + ekgk::MFMA_PAD, L.n_chunks, L.n_bricks, L.n_classes};
+}
+
+// Class sums of one request in the fixed workspace: a row per window piece
+// and class of the window, three sums per lead slot.  The launches divide
+// whatever that comes to among the 16-lead rows, so that the batch that fits
+// depends on this figure alone.
+int64_t fixed_class_bytes(const ReqSpec& r, int LP)
+{
+    const EcgLayout& L = r.h->layout;
+    return L.n_classes > 0 ? (int64_t)L.n_cpieces[r.nhood] * CLASS_WINDOW * (3 * LP * 8 + 8) : 0;
 }
 
 template <class T>
@@ -799,6 +891,7 @@ void append(std::vector<char>& buf, const T* p, size_t n)
 size_t group_device_bytes(const GroupPlan& g)
 {
     size_t s = 0;
+    int64_t gsum = 0, line_max = 0;
     const int LP = g.LP;
     for (const ReqSpec& r : g.reqs) {
         const EcgLayout& L = r.h->layout;
@@ -807,34 +900,27 @@ size_t group_device_bytes(const GroupPlan& g)
         const bool fits = L.valid && (L.class_min == 0 || g.mfma);
         const int64_t est = std::max<int64_t>(1, V / 64 + r.h->max_layer + 4);
         const int64_t nmix = fits ? L.n_chunks : est;
-        // sums rows: the chunks outside classes and, on the matrix-core path,
-        // CLASS_WINDOW per class-window piece (exact once the cells are
-        // built; before that bounded by a piece per window and one per
-        // CLASS_PIECE groups of at most 9 entries per class voxel)
-        int64_t pieces = 0;
         if (g.mfma && fits && L.n_classes > 0) {
-            if (L.cells_built[g.nhood]) {
-                pieces = L.n_cpieces[g.nhood];
-            } else {
-                int64_t cv = 0;
-                for (const int4& cc : L.h_cchunks) cv += cc.z - cc.y;
-                pieces = (L.n_classes + CLASS_WINDOW - 1) / CLASS_WINDOW + (9 * cv / 16 + CLASS_PIECE - 1) / CLASS_PIECE;
-            }
+            // lines of class sums (before the cells are built: each class in
+            // an eighth of the regions)
+            const int64_t lines = L.cells_built[g.nhood] ? L.n_lines[g.nhood] : (int64_t)8 * L.n_classes;
+            gsum += lines * r.L * 8;
+            line_max = std::max(line_max, lines);
         }
-        const int64_t nall = fits ? (int64_t)L.n_chunks + pieces * CLASS_WINDOW : est;
         const int64_t ncls = fits ? L.n_classes : 0;
         const int64_t rows = g.mfma ? 0 : V + ekgk::MFMA_PAD;
         s += (size_t)r.nl * 9 * 8 + (size_t)r.L * 3 * 8 + (size_t)r.Tp * 16;
         s += (size_t)r.nl * (sizeof(ekgk::LayerConst) + r.Tp * 16);
         s += (size_t)rows * (16 * 8 + 16);
-        s += (size_t)nall * (3 * LP * 8 + 8) + (size_t)ncls * 3 * LP * 8;
+        s += (size_t)nmix * (3 * LP * 8 + 8) + (size_t)ncls * 3 * LP * 8;
         s += (size_t)r.nl * ((r.Tp >> (g.mfma ? ekgk::BT_SHIFT_MFMA : ekgk::BT_SHIFT_VALU)) + 1) *
              (8 + 2 * LP * 8);
         s += (size_t)nmix * LP * r.Tp * 8;
         s += (size_t)r.L * r.T * 8;
-        s += sizeof(ekgk::ReqDev) + sizeof(ekgk::HeartDev) + 9 * 8;  // record, heart, nine start tables
+        // record, heart, six start tables, class rows
+        s += sizeof(ekgk::ReqDev) + sizeof(ekgk::HeartDev) + 6 * 8 + sizeof(ekgk::ClassSeg) + r.L * 12;
     }
-    return s;
+    return s + (size_t)std::max(line_max * LINE_BYTES, std::min(gsum + line_max * LINE_BYTES, GSUM_BYTES));
 }
 
 void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, const double* d_k,
@@ -865,7 +951,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     std::vector<std::pair<std::pair<double, double>, std::pair<int64_t, int64_t>>> grids;  // (start, dt) -> (Tp, off)
     std::vector<int64_t> st_red(B + 1, 0);
     std::vector<int64_t> st_lf(B + 1, 0), st_ch(B + 1, 0), st_xy(B + 1, 0), st_lay(B + 1, 0), st_out(B + 1, 0),
-        st_cc(B + 1, 0), st_cs(B + 1, 0), st_cl(B + 1, 0);
+        st_cs(B + 1, 0), st_cl(B + 1, 0);
     int64_t k_off = 0, pos_off = 0, rows = 0, c_off = 0, p_off = 0, pre_off = 0;
     if (!dev_in) {
         ws.h_k.clear();
@@ -883,10 +969,18 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
             hi = (int)hs.size();
             hs.push_back(&h);
             ekgk::HeartDev d = h.layout.dev;
-            d.cgrp = g.mfma ? h.layout.cgrp[g.nhood].as<float>() : nullptr;
-            d.crow = g.mfma ? h.layout.crow[g.nhood].as<int2>() : nullptr;
-            d.cpieces = g.mfma ? h.layout.cpieces[g.nhood].as<int4>() : nullptr;
-            d.cwin = g.mfma ? h.layout.cwin[g.nhood].as<int>() : nullptr;
+            if (g.mfma) {
+                const EcgLayout& hl = h.layout;
+                d.cregion = hl.cregion[g.nhood].as<int4>();
+                d.cbox = hl.cbox[g.nhood].as<int4>();
+                d.cinit = hl.cinit[g.nhood].as<int4>();
+                d.ccoef = hl.ccoef[g.nhood].as<int4>();
+                d.cmask = hl.cmask[g.nhood].as<uint64_t>();
+                d.cs_off = hl.cs_off[g.nhood].as<int>();
+                d.cs_line = hl.cs_line[g.nhood].as<int>();
+                d.n_lines = hl.n_lines[g.nhood];
+                d.n_regions = hl.n_regions[g.nhood];
+            }
             hdev.push_back(d);
         }
         int64_t t_off = -1;
@@ -933,11 +1027,10 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         }
         rows += z.rows;
         c_off += z.chunks;
-        p_off += z.mixed * LP * q.Tp;
+        p_off += z.chunks * LP * q.Tp;
         pre_off += (int64_t)q.nl * ((q.Tp >> R.bt_shift) + 1);
         st_lf[r + 1] = st_lf[r] + z.bricks;
-        st_ch[r + 1] = st_ch[r] + z.mixed;
-        st_cc[r + 1] = st_cc[r] + z.cchunks;
+        st_ch[r + 1] = st_ch[r] + z.chunks;
         st_xy[r + 1] = st_xy[r] + (int64_t)q.nl * q.Tp;
         st_lay[r + 1] = st_lay[r] + q.nl;
         st_out[r + 1] = st_out[r] + (int64_t)q.L * q.T;
@@ -948,8 +1041,9 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         st_cs[r + 1] = st_cs[r] + z.classes;
         st_cl[r + 1] = st_cl[r] + (z.classes > 0 ? q.n_tiles : 0);
     }
-    if (st_lf[B] > 0x7fffffffLL || st_ch[B] > 0x7fffffffLL || st_lay[B] > 0x7fffffffLL || st_cc[B] > 0x7fffffffLL ||
-        st_cl[B] > 0x7fffffffLL)
+    const int64_t pos_max = rd[B - 1].pos_off + 3 * 16;
+    if (st_lf[B] > 0x7fffffffLL || st_ch[B] > 0x7fffffffLL || st_lay[B] > 0x7fffffffLL ||
+        st_cl[B] > 0x7fffffffLL || pos_max > 0x7fffffffLL)
         fail(EKG_EINVAL, "launch group too large");
     // device buffers (grow-only)
     ws.need(ws.lc, (size_t)st_lay[B] * sizeof(ekgk::LayerConst));
@@ -966,17 +1060,61 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         ws.need(ws.ecg, (size_t)std::max<int64_t>(1, st_out[B]) * 8);
         d_ecg = ws.ecg.as<double>();
     }
-    // class-window blocks: runs of consecutive requests of one heart (a
-    // server group is ordered by heart), piece-major within a run
-    std::vector<int4> runs;
-    std::vector<int64_t> st_run(1, 0);
-    if (g.mfma && st_cc[B] > 0) {
+    // Class boxes: the leads of consecutive requests of one heart (a server
+    // group is ordered by heart) fill rows of 16, those of a heart's run cut into
+    // segments whose sums fit gsum, and the segments into launches.
+    std::vector<ekgk::ClassSeg> segs;
+    std::vector<ekgk::ClassLaunch> launches;
+    std::vector<int> rowtab, rowpos, rgseg;
+    if (g.mfma && st_cs[B] > 0) {
+        int64_t need_lines = 0, one_row = 0, fixed = 0;
+        for (int r = 0; r < B; ++r) {
+            const EcgLayout& hl = g.reqs[r].h->layout;
+            if (hl.n_classes == 0) continue;
+            need_lines += (int64_t)g.reqs[r].L * hl.n_lines[g.nhood] / 16 + hl.n_lines[g.nhood];
+            one_row = std::max<int64_t>(one_row, hl.n_lines[g.nhood]);
+            fixed += fixed_class_bytes(g.reqs[r], LP);
+        }
+        const int64_t cap = std::max(one_row, ws.arena ? fixed / LINE_BYTES : std::min(need_lines, GSUM_BYTES / LINE_BYTES));
+        ws.need(ws.gsum, (size_t)(cap * LINE_BYTES));
+        int64_t block0 = 0, used = cap;  // lines taken in the current launch
         for (int r = 0; r < B;) {
-            int r1 = r + 1;
-            while (r1 < B && g.reqs[r1].h == g.reqs[r].h) ++r1;
-            const int64_t np = st_cc[r + 1] - st_cc[r];
-            runs.push_back(int4{r, r1 - r, (int)np, 0});
-            st_run.push_back(st_run.back() + np * (r1 - r));
+            const EcgLayout& hl = g.reqs[r].h->layout;
+            int r1 = r;
+            const int rg_first = (int)rgseg.size();
+            for (; r1 < B && g.reqs[r1].h == g.reqs[r].h; ++r1)
+                if (hl.n_classes > 0)
+                    for (int i = 0; i < g.reqs[r1].L; ++i) {
+                        rowtab.push_back(r1 << 5 | i);
+                        rowpos.push_back((int)rd[r1].pos_off + 3 * i);
+                    }
+            while (rowtab.size() & 15) {
+                rowtab.push_back(rowtab.back() | (int)0x80000000u);
+                rowpos.push_back(rowpos.back());
+            }
+            const int64_t lines = std::max(1, hl.n_lines[g.nhood]);
+            const int rg_end = (int)(rowtab.size() / 16);
+            for (int rg = rg_first; rg < rg_end;) {
+                if (used + lines > cap || launches.back().n_rg >= 65535) {
+                    launches.push_back(ekgk::ClassLaunch{(int)segs.size(), 0, rg, 0, 0});
+                    used = 0;
+                }
+                ekgk::ClassLaunch& la = launches.back();
+                const int n = (int)std::min<int64_t>({rg_end - rg, (cap - used) / lines, 65535 - la.n_rg});
+                const int nr = hl.n_regions[g.nhood];
+                // rows a block: as many as leave about six rounds of blocks on
+                // the chip (three a CU), at most 8
+                const int per = (int)std::max<int64_t>(1, std::min<int64_t>(8, (int64_t)n * nr / (6 * 768)));
+                segs.push_back(ekgk::ClassSeg{rg, n, nr, rd[r].heart, per, 0, block0, used});
+                for (int i = 0; i < n; ++i) rgseg.push_back((int)segs.size() - 1);
+                const int64_t nblk = (int64_t)nr * ((n + per - 1) / per);
+                block0 += nblk;
+                la.blocks += nblk;
+                ++la.n_segs;
+                la.n_rg += n;
+                used += n * lines;
+                rg += n;
+            }
             r = r1;
         }
     }
@@ -987,13 +1125,16 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     const size_t o_req = tables.size();
     append(tables, rd.data(), rd.size());
     const size_t o_st = tables.size();
-    for (auto* st : {&st_lf, &st_ch, &st_xy, &st_lay, &st_out, &st_cc, &st_cs, &st_cl, &st_red})
+    for (auto* st : {&st_lf, &st_ch, &st_xy, &st_lay, &st_cl, &st_red})
         append(tables, st->data(), st->size());
-    const size_t o_rst = tables.size();
-    append(tables, st_run.data(), st_run.size());
-    tables.resize((tables.size() + 15) & ~(size_t)15);  // int4 alignment
-    const size_t o_runs = tables.size();
-    append(tables, runs.data(), runs.size());
+    const size_t o_seg = tables.size();
+    append(tables, segs.data(), segs.size());
+    const size_t o_rgseg = tables.size();
+    append(tables, rgseg.data(), rgseg.size());
+    const size_t o_row = tables.size();
+    append(tables, rowtab.data(), rowtab.size());
+    const size_t o_pos = tables.size();
+    append(tables, rowpos.data(), rowpos.size());
     void* before = ws.hearts.p;
     ws.need(ws.hearts, tables.size());
     if (ws.hearts.p != before) ws.h_tables.clear();
@@ -1041,12 +1182,8 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     a.ch_start = stp + (B + 1);
     a.xy_start = stp + 2 * (B + 1);
     a.lay_start = stp + 3 * (B + 1);
-    a.out_start = stp + 4 * (B + 1);
-    a.cs_start = stp + 6 * (B + 1);
-    a.cl_start = stp + 7 * (B + 1);
-    a.red_start = stp + 8 * (B + 1);
-    a.n_cc = st_cc[B];
-    a.n_cs = st_cs[B];
+    a.cl_start = stp + 4 * (B + 1);
+    a.red_start = stp + 5 * (B + 1);
     a.cs_max = 0;
     for (int r = 0; r < B; ++r) a.cs_max = std::max<int>(a.cs_max, (int)(st_cs[r + 1] - st_cs[r]));
     a.n_cl = st_cl[B];
@@ -1057,16 +1194,16 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     for (int r = 1; r < B && a.ch_uniform; ++r)
         if (st_ch[r + 1] - st_ch[r] != a.ch_uniform) a.ch_uniform = 0;
     a.one_heart = hs.size() == 1 ? 1 : 0;
-    a.cc_runs = reinterpret_cast<const int4*>(tb + o_runs);
-    a.cc_rstart = reinterpret_cast<const int64_t*>(tb + o_rst);
-    a.n_runs = (int)runs.size();
+    a.segs = reinterpret_cast<const ekgk::ClassSeg*>(tb + o_seg);
+    a.rgseg = reinterpret_cast<const int*>(tb + o_rgseg);
+    a.rowtab = reinterpret_cast<const int*>(tb + o_row);
+    a.rowpos = reinterpret_cast<const int*>(tb + o_pos);
     // class-kernel blocks: XCD-aware order when every request has the same count
     a.cl_per_req = (B > 0 && B % 8 == 0) ? (int)(st_cl[1] - st_cl[0]) : 0;
     for (int r = 1; r < B && a.cl_per_req; ++r)
         if (st_cl[r + 1] - st_cl[r] != a.cl_per_req) a.cl_per_req = 0;
     a.n_xy = st_xy[B];
     a.n_lay = st_lay[B];
-    a.n_out = st_out[B];
     a.n_red = st_red[B];
     a.layer_k = d_k;
     a.lead_pos = d_pos;
@@ -1081,10 +1218,11 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     a.pre_rng = ws.pre_rng.as<int2>();
     a.pre_ab = ws.pre_ab.as<double>();
     a.partial = ws.partial.as<double>();
+    a.gsum = ws.gsum.as<double>();
     a.csums = ws.csums.as<double>();
     a.ecg = d_ecg;
     auto launch_all = [&](bool timed) {
-        // The timed kernel is the dominant one of each path: the class-window
+        // The timed kernel is the dominant one of each path: the class-box
         // kernel, or without classes the chunk kernel (matrix-core path), or
         // the fused transition-tile kernel (vector ALUs).
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1099,11 +1237,18 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
             hip_check(hipEventRecord(e1, stream), "hipEventRecord");
             ctx.pending.emplace_back(e0, e1);
         };
-        if (g.mfma && a.n_cc > 0 && ws.side) {
-            // Two branches: the class-window kernel and the class sums on
+        auto classes = [&]() {
+            for (const ekgk::ClassLaunch& c : launches) {
+                if (&c == &launches[0]) tic();
+                hip_check(ekgk::launch_class_boxes(a, c, stream), "class_box launch");
+                if (&c == &launches[0]) toc();
+                hip_check(ekgk::launch_class_sums(a, c, stream), "class_sums launch");
+            }
+        };
+        if (g.mfma && !launches.empty() && ws.side) {
+            // Two branches: the class-box kernel and the class sums on
             // `stream`, beside the AP tables, chunk, prefix and reduction
-            // kernels on the side stream (they share no buffer: the chunk
-            // and class-window kernels write disjoint rows of the sums); the
+            // kernels on the side stream (they share no buffer); the
             // class ECG kernel adds to the reduction's output after both.
             hip_check(hipEventRecord(ws.ev_fork, stream), "hipEventRecord");
             hip_check(hipStreamWaitEvent(ws.side, ws.ev_fork, 0), "hipStreamWaitEvent");
@@ -1112,24 +1257,18 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
             hip_check(ekgk::launch_layer_prefix(a, ws.side), "layer_prefix launch");
             hip_check(ekgk::launch_ecg_reduce(a, ws.side), "ecg_reduce launch");
             hip_check(hipEventRecord(ws.ev_join, ws.side), "hipEventRecord");
-            tic();
-            hip_check(ekgk::launch_class_windows(a, stream), "class_window launch");
-            toc();
-            hip_check(ekgk::launch_class_sums(a, stream), "class_sums launch");
+            classes();
             hip_check(hipStreamWaitEvent(stream, ws.ev_join, 0), "hipStreamWaitEvent");
             hip_check(ekgk::launch_ecg_class(a, stream), "ecg_class launch");
             return;
         }
         hip_check(ekgk::launch_ap_tables(a, stream), "ap_tables launch");
         if (g.mfma) {
-            // the class-window kernel is timed when the group has classes
-            if (a.n_cc == 0) tic();
+            // the class-box kernel is timed when the group has classes
+            if (launches.empty()) tic();
             hip_check(ekgk::launch_ecg_chunk(a, stream), "ecg_chunk launch");
-            if (a.n_cc == 0) toc();
-            if (a.n_cc > 0) tic();
-            hip_check(ekgk::launch_class_windows(a, stream), "class_window launch");
-            if (a.n_cc > 0) toc();
-            hip_check(ekgk::launch_class_sums(a, stream), "class_sums launch");
+            if (launches.empty()) toc();
+            classes();
             hip_check(ekgk::launch_layer_prefix(a, stream), "layer_prefix launch");
         } else {
             hip_check(ekgk::launch_lead_field(a, stream), "lead_field launch");
@@ -1151,6 +1290,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     // per-request values live in device tables and buffers, so new inputs
     // in the same places need no recapture.  The graph holds kernels only.
     std::vector<char> key(reinterpret_cast<const char*>(&a), reinterpret_cast<const char*>(&a) + sizeof a);
+    append(key, launches.data(), launches.size());
     if (!ws.graph || key != ws.graph_key) {
         if (ws.graph) {
             (void)hipGraphExecDestroy(ws.graph);

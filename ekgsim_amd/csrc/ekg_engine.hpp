@@ -42,7 +42,7 @@ struct DevBuf {
 // Device workspace of one launch group on one stream (grow-only buffers).
 struct Workspace {
     DevBuf hearts, reqs, starts, layer_k, lead_pos, tgrid, thl, lc, xy, G, aux, sums, bnd, pre_rng,
-        pre_ab, partial, csums, ecg;
+        pre_ab, partial, gsum, csums, ecg;
     std::vector<double> h_k, h_pos, h_tgrid;
     std::vector<float> h_thl;
     std::vector<char> h_tables;    // hearts + reqs + starts as last uploaded
@@ -106,13 +106,13 @@ struct EcgLayout {
     std::vector<double> h_class_a;
     std::vector<uint2> h_geo;      // per voxel of the layout: packed grid coordinates, 3x3x3 myocardium mask
     // Per dipole neighbourhood (EKG_NHOOD_*), built on first use: the class
-    // windows' entries as lane-major groups of 16 and their pieces (see
-    // ensure_cells).  n_ccells counts (class, cell) pairs with a non-zero
-    // dipole vector, n_centries (window, cell) pairs.
+    // boxes and their regions (see ensure_cells).  n_ccells counts (class,
+    // cell) pairs with a non-zero dipole vector; n_centries and n_cpieces
+    // are the sizes of the layout in windows of six classes (layout_info).
     bool cells_built[4] = {false, false, false, false};
-    int64_t n_ccells[4] = {0, 0, 0, 0}, n_centries[4] = {0, 0, 0, 0}, n_cgroups[4] = {0, 0, 0, 0};
-    int n_cpieces[4] = {0, 0, 0, 0};
-    DevBuf cgrp[4], crow[4], cpieces[4], cwin[4];
+    int64_t n_ccells[4] = {0, 0, 0, 0}, n_centries[4] = {0, 0, 0, 0};
+    int n_cpieces[4] = {0, 0, 0, 0}, n_lines[4] = {0, 0, 0, 0}, n_regions[4] = {0, 0, 0, 0};
+    DevBuf cregion[4], cbox[4], cinit[4], ccoef[4], cmask[4], cs_off[4], cs_line[4];
     std::vector<int> h_layer_chunk;
     std::vector<double> h_layer_t0;
     DevBuf vox_chunk, vox_a64, vox_a, vox_geo, chunks, bricks, brick_off, brick_vox, halo_off, halo_cells,

@@ -23,16 +23,10 @@ constexpr int CHUNK_MAX = 512;
 // launch), 64 on the vector-ALU path (one step per lane of a wave).
 constexpr int BT_SHIFT_MFMA = 3;
 constexpr int BT_SHIFT_VALU = 6;
-// Activation classes per class window, and groups of 16 window entries per
-// piece (one class-window block per piece and request).  Six classes keep the
-// kernel's accumulators within 64 VGPRs (eight waves per SIMD); eight share
-// more lead weights but leave five waves and run slower.
-constexpr int CLASS_WINDOW = 6;
-// Largest class-window piece (groups of 16 entries); a window is cut into
-// the fewest pieces of at most this size, all of about equal size.  Measured
-// per 256 x 12 step on the 128^3 heart: 1.46 ms at 1024 against 1.48-1.49 ms
-// with 512 (equal or fixed pieces), 1.49 ms at 1536 and 1.54 ms at 2048.
-constexpr int CLASS_PIECE = 1024;
+// Class boxes (ecg_class_box_kernel): waves per block, most classes of a
+// region (LDS rows of 16 leads per wave: 12.4 KB, so that three blocks share a CU).
+constexpr int CB_WAVES = 4;
+constexpr int CB_SLOTS = 96;
 
 // ---- excitation sequence ---------------------------------------------------
 
@@ -81,17 +75,21 @@ struct HeartDev {
     const int4* cchunks;         // [n_cchunks] {layer, v_begin, v_end, t_ref as float bits}
     const int4* classes;         // [n_classes] {layer, first class chunk, end class chunk, 0}
     const double* class_a;       // [n_classes] activation time of the class
-    // class windows for the group's neighbourhood: CLASS_WINDOW classes each
-    // (window w: classes [w CLASS_WINDOW, (w+1) CLASS_WINDOW)), their entries
-    // (cells with a non-zero dipole vector for a class of the window) in
-    // groups of 16, group q in rows crow[q].x, ... of 64 floats of cgrp
-    // {coordinate, |c|^2, then a coefficient row per class of the mask
-    // crow[q].y}; the groups cut into pieces {window, first group, end group},
-    // those of window w being [cwin[w], cwin[w+1])
-    const float* cgrp;
-    const int2* crow;
-    const int4* cpieces;
-    const int* cwin;
+    // class boxes for the group's neighbourhood (ensure_cells): regions
+    // {first box, end box, first line, lines} and {first | last << 16 cell + 1
+    // per axis}; per box 64 records (its tiles of 4 classes {sub-bricks, 4 slot bytes,
+    // first block, 0}, from 16 on {tiles, rows of 16 cells in use, 0, 0} and {first
+    // cell + 1}) and the 16 tiles' 16 accumulator starts; coefficient blocks of 64
+    // lanes x 16 bytes; per box and sub-brick the cells that carry dipoles; the lines
+    // (region, slot) of class k are cs_line[cs_off[k] .. cs_off[k + 1])
+    const int4* cregion;
+    const int4* cbox;
+    const int4* cinit;
+    const int4* ccoef;
+    const uint64_t* cmask;
+    const int* cs_off;
+    const int* cs_line;
+    int n_lines, n_regions;
     int n0, n1, n2;
     int V, n_chunks, n_bricks, max_layer;
     int n_cchunks, n_classes;
@@ -114,6 +112,21 @@ struct ReqDev {
     int64_t cls_off;  // class sums: csums[(cls_off + class)*3*LP ...]
 };
 
+// A segment of the class-box launches: the 16-lead rows [rg0, rg0 + n_rg) of
+// consecutive requests of one heart, all its regions; `per` rows a block,
+// blocks n_regions x ceil(n_rg / per) from block0 on, sums at line
+// goff + (row - rg0) n_lines of gsum.
+struct ClassSeg {
+    int rg0, n_rg, n_regions, heart, per, pad;
+    int64_t block0, goff;
+};
+// One launch of the class-box and class-sum kernels: segments whose sums fit
+// gsum together.
+struct ClassLaunch {
+    int seg0, n_segs, rg0, n_rg;
+    int64_t blocks;
+};
+
 // A launch group: requests of any hearts, lead counts and time grids that
 // share the dipole neighbourhood, the padded lead count LP and the kernel
 // path.  Work-item starts are exclusive prefix sums over requests (B + 1).
@@ -128,19 +141,17 @@ struct GroupArgs {
     const int64_t* ch_start;   // chunks per request
     const int64_t* xy_start;   // nl * Tp per request
     const int64_t* lay_start;  // nl per request
-    const int64_t* out_start;  // L * T per request
-    const int64_t* cs_start;   // activation classes per request
     const int64_t* cl_start;   // 64-step tiles of the class kernel per request (0 without classes)
     const int64_t* red_start;  // reduction items per request: L x (T rounded up to a bound tile)
-    int64_t n_lf, n_ch, n_xy, n_lay, n_out, n_cc, n_cs, n_cl, n_red;  // totals
+    int64_t n_lf, n_ch, n_xy, n_lay, n_cl, n_red;  // totals
     int ch_uniform;            // chunks per request when all requests have the same count, else 0
     int one_heart;             // every request on one heart (tables hold it as heart 0)
-    // class-window blocks: runs of consecutive requests of one heart
-    // {first request, requests, pieces of the heart}, blocks of run u
-    // [cc_rstart[u], cc_rstart[u+1]) = pieces x requests
-    const int4* cc_runs;
-    const int64_t* cc_rstart;
-    int n_runs;
+    // class boxes: segments, per 16-lead row its segment, and per lead of it
+    // request << 5 | lead (bit 31: a repeat that fills the last row of a segment's requests)
+    const ClassSeg* segs;
+    const int* rgseg;
+    const int* rowtab;
+    const int* rowpos;         // electrode offsets of the same rows (lead_pos[rowpos + c])
     int cl_per_req;            // class-kernel blocks per request when equal for all and B % 8 == 0, else 0
     const double* layer_k;
     const double* lead_pos;
@@ -155,6 +166,7 @@ struct GroupArgs {
     int2* pre_rng;             // per (request, layer, bound tile): transition chunks [lo, hi)
     double* pre_ab;            // per (request, layer, bound tile): [2][LP]; tile n_bt: [LP] sum G
     double* partial;
+    double* gsum;              // class boxes: [line][16 leads] sum G per region and class
     double* csums;             // per (request, class): [3][LP] sum G, sum G P', sum G Q'
     double* ecg;
 };
@@ -169,10 +181,10 @@ hipError_t launch_ecg_chunk(const GroupArgs& a, hipStream_t s);
 hipError_t launch_ecg_reduce(const GroupArgs& a, hipStream_t s);
 // Resolves every matrix-core-path kernel once (see ekg_ecg.hip).
 void prime_kernels();
-// Activation classes: the lead-weight sums of the class chunks, their sums
+// Activation classes: the lead-weight sums per region and class, the sums
 // per class, then the classes' terms added to the reduced ECG.
-hipError_t launch_class_windows(const GroupArgs& a, hipStream_t s);
-hipError_t launch_class_sums(const GroupArgs& a, hipStream_t s);
+hipError_t launch_class_boxes(const GroupArgs& a, const ClassLaunch& c, hipStream_t s);
+hipError_t launch_class_sums(const GroupArgs& a, const ClassLaunch& c, hipStream_t s);
 hipError_t launch_ecg_class(const GroupArgs& a, hipStream_t s);
 
 // ---- fixed workspace of the allocation-free entry point ----------------------
