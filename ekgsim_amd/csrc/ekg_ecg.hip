@@ -513,21 +513,56 @@ __global__ __launch_bounds__(256) void chunk_sums_kernel(
 // (at most PRE_SEGS segments), each summed in chunk order; the segment sums
 // are accumulated in order; a prefix at lo is the accumulated sum of the
 // segments before lo's segment plus that segment's chunks before lo, in order.
+//
+// Latency bound: chains of dependent loads in few blocks.  So a block
+// has 1024 threads where a layer has many chunks (the segment sums are then a few loads
+// deep), the range of a tile is searched once, not once per lead, and a
+// search takes two steps for every load it waits for (three probes at a time).
+// 64 x 12 leads on the 128^3 conduction-matrix heart (1,000 chunks a layer):
+// 95 us with 256 threads, a search per (tile, lead) and one probe at a time, 45 us so.
 constexpr int PRE_SEGS = 128;
 
+// First index in [lo, hi) whose value (x: the chunk's first tile not skipped, y:
+// its first saturated tile) exceeds `tile`; the values are non-decreasing.
+template <bool Y>
+__device__ __forceinline__ int first_above(const int2* __restrict__ bd, int lo, int hi, int tile)
+{
+    while (hi - lo > 0) {
+        // probes at the quarters: up to three loads in flight
+        const int n = hi - lo, m1 = lo + (n >> 2), m2 = lo + (n >> 1), m3 = lo + (3 * n >> 2);
+        const int v1 = Y ? bd[m1].y : bd[m1].x, v2 = Y ? bd[m2].y : bd[m2].x, v3 = Y ? bd[m3].y : bd[m3].x;
+        if (v2 <= tile) {
+            if (v3 <= tile)
+                lo = m3 + 1;
+            else {
+                lo = m2 + 1;
+                hi = m3;
+            }
+        } else {
+            if (v1 <= tile) {
+                lo = m1 + 1;
+                hi = m2;
+            } else
+                hi = m1;
+        }
+    }
+    return lo;
+}
+
 template <int LP>
-__global__ __launch_bounds__(256) void layer_prefix_kernel(
+__global__ __launch_bounds__(1024) void layer_prefix_kernel(
     const HeartDev* __restrict__ hearts, const ReqDev* __restrict__ reqs, int B,
     const int64_t* __restrict__ lay_start, const double* __restrict__ sums,
     const int2* __restrict__ bnd, int2* __restrict__ pre_rng, double* __restrict__ pre_ab)
 {
     constexpr int NC3 = 3 * LP;
     __shared__ double s_seg[PRE_SEGS + 1][NC3];   // [k][col]: sum of the segments before k
+    __shared__ int s_lo[1024];                    // lo of the tiles of one round
     const int r = find_req(lay_start, B, blockIdx.x);
     const ReqDev R = reqs[r];
     const HeartDev& H = hearts[R.heart];
     const int l = (int)(blockIdx.x - lay_start[r]) + 1;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, nt = blockDim.x;
     const int cb = l <= H.max_layer ? H.layer_chunk[l] : 0;
     const int ce = l <= H.max_layer ? H.layer_chunk[l + 1] : 0;
     const int nc = ce - cb;
@@ -538,53 +573,49 @@ __global__ __launch_bounds__(256) void layer_prefix_kernel(
     const int2* bd = bnd + R.c_off;
     const double* sc = sums + R.c_off * NC3;
     // segment sums (columns: sum G, sum G P', sum G Q' per lead)
-    for (int it = t; it < nseg * NC3; it += blockDim.x) {
+    for (int it = t; it < nseg * NC3; it += nt) {
         const int k = it / NC3, col = it - k * NC3;
         const int c0 = cb + k * seg, c1 = c0 + seg < ce ? c0 + seg : ce;
         double acc = 0.0;
+#pragma unroll 4
         for (int c = c0; c < c1; ++c) acc += sc[(int64_t)c * NC3 + col];
         s_seg[k + 1][col] = acc;
     }
-    __syncthreads();
-    if (t < NC3) {
-        double run = 0.0;
-        s_seg[0][t] = 0.0;
-        for (int k = 1; k <= nseg; ++k) {
-            run += s_seg[k][t];
-            s_seg[k][t] = run;
+    for (int t0 = 0; t0 < nbt; t0 += nt) {
+        // the tiles' ranges, one search a thread
+        if (t0 + t < nbt) {
+            const int lo = first_above<true>(bd, cb, ce, t0 + t);
+            s_lo[t] = lo;
+            pre_rng[slot + t0 + t] = int2{lo, first_above<false>(bd, lo, ce, t0 + t)};
         }
-    }
-    __syncthreads();
-    // per (tile, lead): transition range by binary searches, prefix at lo
-    for (int it = t; it < nbt * LP; it += blockDim.x) {
-        const int tile = it / LP, i = it - tile * LP;
-        int a0 = cb, a1 = ce;
-        while (a0 < a1) {
-            const int mid = (a0 + a1) >> 1;
-            if (bd[mid].y <= tile)
-                a0 = mid + 1;
-            else
-                a1 = mid;
+        __syncthreads();
+        if (t0 == 0) {
+            if (t < NC3) {
+                double run = 0.0;
+                s_seg[0][t] = 0.0;
+#pragma unroll 8
+                for (int k = 1; k <= nseg; ++k) {
+                    run += s_seg[k][t];
+                    s_seg[k][t] = run;
+                }
+            }
+            __syncthreads();
         }
-        const int lo = a0;
-        a1 = ce;
-        while (a0 < a1) {
-            const int mid = (a0 + a1) >> 1;
-            if (bd[mid].x <= tile)
-                a0 = mid + 1;
-            else
-                a1 = mid;
+        // per (tile, lead): the prefix at lo
+        const int n_t = nbt - t0 < nt ? nbt - t0 : nt;
+        for (int it = t; it < n_t * LP; it += nt) {
+            const int tile = it / LP, i = it - tile * LP;
+            const int lo = s_lo[tile], k = (lo - cb) / seg;
+            double A = s_seg[k][LP + i], Bq = s_seg[k][2 * LP + i];
+#pragma unroll 4
+            for (int c = cb + k * seg; c < lo; ++c) {
+                A += sc[(int64_t)c * NC3 + LP + i];
+                Bq += sc[(int64_t)c * NC3 + 2 * LP + i];
+            }
+            pre_ab[(slot + t0 + tile) * 2 * LP + i] = A;
+            pre_ab[(slot + t0 + tile) * 2 * LP + LP + i] = Bq;
         }
-        const int hi = a0;
-        const int k = (lo - cb) / seg;
-        double A = s_seg[k][LP + i], Bq = s_seg[k][2 * LP + i];
-        for (int c = cb + k * seg; c < lo; ++c) {
-            A += sc[(int64_t)c * NC3 + LP + i];
-            Bq += sc[(int64_t)c * NC3 + 2 * LP + i];
-        }
-        if (i == 0) pre_rng[slot + tile] = int2{lo, hi};
-        pre_ab[(slot + tile) * 2 * LP + i] = A;
-        pre_ab[(slot + tile) * 2 * LP + LP + i] = Bq;
+        __syncthreads();
     }
     if (t < LP) {
         pre_ab[(slot + nbt) * 2 * LP + t] = s_seg[nseg][t];
@@ -1156,11 +1187,12 @@ __global__ __launch_bounds__(1024) void ecg_chunk_kernel(
 // Reduction
 // ---------------------------------------------------------------------------
 
-// ecg[r][i][t] for t < Tn: per layer (in order) the closed form of the
-// chunks saturated by t's tile, X_l(t) A + Y_l(t) B, then k0 * sum G, then
-// the partial rows of the chunks in transition in chunk order; 0 for
-// Tn <= t < T: samples past the last iteration of the reference's neighbour
-// loop (simulator.cpp:519) receive no dipole.
+// ecg[r][i][t] for t < Tn: per layer the closed form of the chunks saturated by
+// t's tile, X_l(t) A + Y_l(t) B, then k0 * sum G, and the partial rows of the
+// chunks in transition; 0 for Tn <= t < T: samples past the last iteration of the
+// reference's neighbour loop (simulator.cpp:519) receive no dipole.
+//
+// ecg_reduce_kernel: one thread per (tile, lead, step).
 template <int LP>
 __global__ void ecg_reduce_kernel(const HeartDev* __restrict__ hearts, const ReqDev* __restrict__ reqs,
                                   int B, const int64_t* __restrict__ red_start, int64_t n_red,
@@ -1211,6 +1243,79 @@ __global__ void ecg_reduce_kernel(const HeartDev* __restrict__ hearts, const Req
             }
         }
         ecg[R.ecg_off + (int64_t)i * R.T + j] = s;
+    }
+}
+
+// ecg_reduce_parts_kernel: the same sums for groups whose tiles have long
+// ranges (the steps of the upstroke: about 1,000 of the 2,900 chunks of the 128^3
+// conduction-matrix heart), which leave the few threads that have them a long chain
+// of loads, eight at a time.  One block per (request, tile): a tile's rows of one
+// chunk are one contiguous run (LP leads x the tile's steps), `w` consecutive threads
+// read whole cache lines of it, and RED_PARTS such sets divide the sum: part p
+// adds, of every layer, the p-th of RED_PARTS contiguous shares of the range, and,
+// of the closed forms, layers p, p + RED_PARTS, ...; the parts are added in order.
+// The shares depend on the tile's ranges only, and the host picks the kernel by
+// the heart and the request's start alone, so a request's bits do not depend on
+// its batch.  64 x 12 leads on that heart: 178 us with one thread a sum, 140 us with
+// four parts, 130 us with eight (0.47 GB of rows, 3.6 TB/s).
+constexpr int RED_PARTS = 8;
+
+template <int LP>
+__global__ void ecg_reduce_parts_kernel(const HeartDev* __restrict__ hearts, const ReqDev* __restrict__ reqs, int B,
+                                        const int64_t* __restrict__ redp_start, const LayerConst* __restrict__ lc,
+                                        const double2* __restrict__ xy, const int2* __restrict__ pre_rng,
+                                        const double* __restrict__ pre_ab, const double* __restrict__ partial,
+                                        double* __restrict__ ecg)
+{
+    extern __shared__ double s_part[];  // [RED_PARTS - 1][items of a round]
+    const int r = find_req(redp_start, B, blockIdx.x);
+    const ReqDev R = reqs[r];
+    const HeartDev& H = hearts[R.heart];
+    const int tile = (int)(blockIdx.x - redp_start[r]);
+    const int bs = R.bt_shift, w = blockDim.x / RED_PARTS;  // items a round
+    const int p = threadIdx.x / w, e0 = threadIdx.x - p * w;
+    const int nbt = R.Tp >> bs;
+    const int nl = R.nl < H.max_layer ? R.nl : H.max_layer;
+    const int64_t st = (int64_t)LP * R.Tp;
+    for (int e = e0; e < (LP << bs); e += w) {  // the same rounds for every thread
+        const int i = e >> bs, j = (tile << bs) + (e & ((1 << bs) - 1));
+        const bool live = i < R.L && j < R.Tn;
+        double s = 0.0;
+        if (live) {
+            const double* pr = partial + R.p_off + prow(i, j, LP, bs);
+            for (int l = 1; l <= nl; ++l) {
+                const int64_t slot = R.pre_off + (int64_t)(l - 1) * (nbt + 1);
+                const int2 rg = pre_rng[slot + tile];
+                if ((l - 1) % RED_PARTS == p) {
+                    const double2 xyj = xy[R.xy_off + (int64_t)(l - 1) * R.Tp + j];
+                    const double* ab = pre_ab + (slot + tile) * 2 * LP;
+                    s = __builtin_fma(xyj.x, ab[i], s);
+                    s = __builtin_fma(xyj.y, ab[LP + i], s);
+                    s = __builtin_fma(lc[R.lay_off + l - 1].k0, pre_ab[(slot + nbt) * 2 * LP + i], s);
+                }
+                // this part's share of the range, eight independent loads
+                // in flight, added in chunk order
+                const int n = rg.y - rg.x;
+                int c = rg.x + n * p / RED_PARTS;
+                const int c1 = rg.x + n * (p + 1) / RED_PARTS;
+                for (; c + 8 <= c1; c += 8) {
+                    double x[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) x[u] = pr[(int64_t)(c + u) * st];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) s += x[u];
+                }
+                for (; c < c1; ++c) s += pr[(int64_t)c * st];
+            }
+        }
+        __syncthreads();
+        if (p > 0) s_part[(p - 1) * w + e0] = s;
+        __syncthreads();
+        if (p == 0 && i < R.L && j < R.T) {
+#pragma unroll
+            for (int q = 0; q < RED_PARTS - 1; ++q) s += s_part[q * w + e0];
+            ecg[R.ecg_off + (int64_t)i * R.T + j] = s;
+        }
     }
 }
 
@@ -1737,7 +1842,7 @@ hipError_t launch_layer_prefix(const GroupArgs& a, hipStream_t s)
     switch (a.LP) {
 #define EKG_PREFIX(LPV)                                                                                  \
     case LPV:                                                                                            \
-        hipLaunchKernelGGL(layer_prefix_kernel<LPV>, dim3((unsigned)a.n_lay), dim3(256), 0, s, a.hearts, \
+        hipLaunchKernelGGL(layer_prefix_kernel<LPV>, dim3((unsigned)a.n_lay), dim3(a.pre_threads), 0, s, a.hearts, \
                            a.reqs, a.B, a.lay_start, a.sums, a.bnd, a.pre_rng, a.pre_ab);               \
         break;
         EKG_PREFIX(4)
@@ -1889,6 +1994,7 @@ static void prime_lp(hipFuncAttributes& at)
     (void)hipFuncGetAttributes(&at, (const void*)class_sums_kernel<LP>);
     (void)hipFuncGetAttributes(&at, (const void*)layer_prefix_kernel<LP>);
     (void)hipFuncGetAttributes(&at, (const void*)ecg_reduce_kernel<LP>);
+    (void)hipFuncGetAttributes(&at, (const void*)ecg_reduce_parts_kernel<LP>);
     (void)hipFuncGetAttributes(&at, (const void*)ecg_class_kernel<LP>);
 }
 
@@ -1905,13 +2011,17 @@ void prime_kernels()
 
 hipError_t launch_ecg_reduce(const GroupArgs& a, hipStream_t s)
 {
-    if (a.n_red == 0) return hipSuccess;
     switch (a.LP) {
 #define EKG_REDUCE(LPV)                                                                                 \
     case LPV:                                                                                           \
-        hipLaunchKernelGGL(ecg_reduce_kernel<LPV>, dim3(grid_for(a.n_red, 256)), dim3(256), 0, s,      \
-                           a.hearts, a.reqs, a.B, a.red_start, a.n_red, a.lc, a.xy, a.pre_rng,          \
-                           a.pre_ab, a.partial, a.ecg);                                                 \
+        if (a.n_redp > 0)                                                                                   \
+            hipLaunchKernelGGL(ecg_reduce_parts_kernel<LPV>, dim3((unsigned)a.n_redp),                       \
+                               dim3(a.red_items * RED_PARTS), a.red_items * (RED_PARTS - 1) * 8, s, a.hearts, \
+                               a.reqs, a.B, a.redp_start, a.lc, a.xy, a.pre_rng, a.pre_ab, a.partial, a.ecg); \
+        if (a.n_red > 0)                                                                                      \
+            hipLaunchKernelGGL(ecg_reduce_kernel<LPV>, dim3(grid_for(a.n_red, 256)), dim3(256), 0, s,         \
+                               a.hearts, a.reqs, a.B, a.red_start, a.n_red, a.lc, a.xy, a.pre_rng,             \
+                               a.pre_ab, a.partial, a.ecg);                                                   \
         break;
         EKG_REDUCE(4)
         EKG_REDUCE(8)

@@ -266,6 +266,7 @@ constexpr int64_t CLASS_PIECE = 1024;
 // and at most 64.
 constexpr int BOX_Z = 4, BOX_Y = 8, BOX_X = 8;
 constexpr int CB_SLOTS = ekgk::CB_SLOTS;
+constexpr int LONG_RANGES = 512;        // chunks from which the reduction sums in parts
 constexpr size_t BOX_CLASSES = 64;  // classes of one listing of a box (16 tiles)
 // Most bytes of class sums per launch; a larger group runs its rows in
 // several launches.
@@ -317,6 +318,8 @@ void ensure_layout(Heart& h, bool mfma)
     const int64_t V = (int64_t)idx.size();
     L.V = V;
     L.max_layer = h.max_layer;
+    L.a_last = 0.0;
+    for (int64_t i : idx) L.a_last = std::max(L.a_last, h.h_act[i]);
     L.h_chunks.clear();
     L.h_cchunks.clear();
     L.h_classes.clear();
@@ -917,8 +920,8 @@ size_t group_device_bytes(const GroupPlan& g)
              (8 + 2 * LP * 8);
         s += (size_t)nmix * LP * r.Tp * 8;
         s += (size_t)r.L * r.T * 8;
-        // record, heart, six start tables, class rows
-        s += sizeof(ekgk::ReqDev) + sizeof(ekgk::HeartDev) + 6 * 8 + sizeof(ekgk::ClassSeg) + r.L * 12;
+        // record, heart, seven start tables, class rows
+        s += sizeof(ekgk::ReqDev) + sizeof(ekgk::HeartDev) + 7 * 8 + sizeof(ekgk::ClassSeg) + r.L * 12;
     }
     return s + (size_t)std::max(line_max * LINE_BYTES, std::min(gsum + line_max * LINE_BYTES, GSUM_BYTES));
 }
@@ -949,7 +952,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     ws.h_tgrid.clear();
     ws.h_thl.clear();
     std::vector<std::pair<std::pair<double, double>, std::pair<int64_t, int64_t>>> grids;  // (start, dt) -> (Tp, off)
-    std::vector<int64_t> st_red(B + 1, 0);
+    std::vector<int64_t> st_red(B + 1, 0), st_redp(B + 1, 0);
     std::vector<int64_t> st_lf(B + 1, 0), st_ch(B + 1, 0), st_xy(B + 1, 0), st_lay(B + 1, 0), st_out(B + 1, 0),
         st_cs(B + 1, 0), st_cl(B + 1, 0);
     int64_t k_off = 0, pos_off = 0, rows = 0, c_off = 0, p_off = 0, pre_off = 0;
@@ -1034,16 +1037,20 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         st_xy[r + 1] = st_xy[r] + (int64_t)q.nl * q.Tp;
         st_lay[r + 1] = st_lay[r] + q.nl;
         st_out[r + 1] = st_out[r] + (int64_t)q.L * q.T;
-        {
-            const int64_t bt = (int64_t)1 << R.bt_shift;
-            st_red[r + 1] = st_red[r] + (int64_t)q.L * ((q.T + bt - 1) / bt) * bt;
-        }
+        const int64_t tiles = ((int64_t)q.T + (1 << R.bt_shift) - 1) >> R.bt_shift;
+        // Long ranges of chunks in transition: a heart of many chunks, from before
+        // its last activation on (a request that starts later meets every
+        // chunk saturated).  512 chunks put about 170 into a range of the upstroke,
+        // where the sums in parts begin to pay (48^3: 157 chunks, 12 us either way).
+        const bool parts = h.layout.n_chunks >= LONG_RANGES && q.start < h.layout.a_last;
+        st_red[r + 1] = st_red[r] + (parts ? 0 : (q.L * tiles) << R.bt_shift);
+        st_redp[r + 1] = st_redp[r] + (parts ? tiles : 0);
         st_cs[r + 1] = st_cs[r] + z.classes;
         st_cl[r + 1] = st_cl[r] + (z.classes > 0 ? q.n_tiles : 0);
     }
     const int64_t pos_max = rd[B - 1].pos_off + 3 * 16;
     if (st_lf[B] > 0x7fffffffLL || st_ch[B] > 0x7fffffffLL || st_lay[B] > 0x7fffffffLL ||
-        st_cl[B] > 0x7fffffffLL || pos_max > 0x7fffffffLL)
+        st_redp[B] > 0x7fffffffLL || st_cl[B] > 0x7fffffffLL || pos_max > 0x7fffffffLL)
         fail(EKG_EINVAL, "launch group too large");
     // device buffers (grow-only)
     ws.need(ws.lc, (size_t)st_lay[B] * sizeof(ekgk::LayerConst));
@@ -1125,7 +1132,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     const size_t o_req = tables.size();
     append(tables, rd.data(), rd.size());
     const size_t o_st = tables.size();
-    for (auto* st : {&st_lf, &st_ch, &st_xy, &st_lay, &st_cl, &st_red})
+    for (auto* st : {&st_lf, &st_ch, &st_xy, &st_lay, &st_cl, &st_red, &st_redp})
         append(tables, st->data(), st->size());
     const size_t o_seg = tables.size();
     append(tables, segs.data(), segs.size());
@@ -1184,6 +1191,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     a.lay_start = stp + 3 * (B + 1);
     a.cl_start = stp + 4 * (B + 1);
     a.red_start = stp + 5 * (B + 1);
+    a.redp_start = stp + 6 * (B + 1);
     a.cs_max = 0;
     for (int r = 0; r < B; ++r) a.cs_max = std::max<int>(a.cs_max, (int)(st_cs[r + 1] - st_cs[r]));
     a.n_cl = st_cl[B];
@@ -1205,6 +1213,15 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     a.n_xy = st_xy[B];
     a.n_lay = st_lay[B];
     a.n_red = st_red[B];
+    a.n_redp = st_redp[B];
+    a.red_items = std::min(128, LP << (g.mfma ? ekgk::BT_SHIFT_MFMA : ekgk::BT_SHIFT_VALU));
+    // a prefix block sums a layer's chunks: wide where there are many (64 requests with
+    // about 1,000 a layer: 10 us less than 256 threads; 128 requests with 130 a layer: 22 us more)
+    int64_t nc_max = 0;
+    for (Heart* hp : hs)
+        for (int l = 1; l <= hp->max_layer; ++l)
+            nc_max = std::max<int64_t>(nc_max, hp->layout.h_layer_chunk[l + 1] - hp->layout.h_layer_chunk[l]);
+    a.pre_threads = nc_max > 512 ? 1024 : 256;
     a.layer_k = d_k;
     a.lead_pos = d_pos;
     a.tgrid = ws.tgrid.as<double>();

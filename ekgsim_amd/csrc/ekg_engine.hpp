@@ -99,6 +99,7 @@ struct EcgLayout {
     int n_chunks = 0;
     int n_bricks = 0;
     int max_layer = 0;
+    double a_last = 0.0;           // latest activation time (0 at least)
     int chunk_target = 0;          // voxels per chunk the layout was cut with
     int class_min = -1;            // smallest class it was built with (0: no classes)
     int n_cchunks = 0, n_classes = 0;

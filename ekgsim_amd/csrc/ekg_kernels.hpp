@@ -143,7 +143,10 @@ struct GroupArgs {
     const int64_t* lay_start;  // nl per request
     const int64_t* cl_start;   // 64-step tiles of the class kernel per request (0 without classes)
     const int64_t* red_start;  // reduction items per request: L x (T rounded up to a bound tile)
-    int64_t n_lf, n_ch, n_xy, n_lay, n_cl, n_red;  // totals
+    const int64_t* redp_start; // bound tiles of the requests with long ranges (none in red_start)
+    int red_items;             // items (lead, step of a tile) of a round of one such tile: LP x steps, at most 128
+    int pre_threads;           // threads of a prefix block
+    int64_t n_lf, n_ch, n_xy, n_lay, n_cl, n_red, n_redp;  // totals
     int ch_uniform;            // chunks per request when all requests have the same count, else 0
     int one_heart;             // every request on one heart (tables hold it as heart 0)
     // class boxes: segments, per 16-lead row its segment, and per lead of it
