@@ -1663,7 +1663,6 @@ void excite(Heart& h, bool is_int, const double* transfer, int rows, int cols, c
     for (int round = 4;; round = std::min(2 * round, MAX_ROUND)) {
         hip_check(hipMemsetAsync(d_any.p, 0, (size_t)round * sizeof(int), s), "hipMemsetAsync");
         for (int q = 0; q < round; ++q) {
-            hip_check(hipMemsetAsync(fb, 0, nbricks, s), "hipMemsetAsync");
             hip_check(ekgk::launch_ca_sweep(is_int, h.d_layer.as<uint8_t>(), d_delay.as<uint8_t>(),
                                             d_wtab.as<double>(), cols, d_dist.p, h.n0, h.n1, h.n2, nb0,
                                             nb1, nb2, fa, fb, d_any.as<int>() + q, s),

@@ -37,7 +37,7 @@ hipError_t launch_ca_init(bool is_int, const uint8_t* layer, const uint8_t* seed
                           uint8_t* active, int n0, int n1, int n2, int nb1, int nb2, hipStream_t s);
 hipError_t launch_ca_sweep(bool is_int, const uint8_t* layer, const uint8_t* delay,
                            const double* wtab, int wcols, void* dist, int n0, int n1, int n2,
-                           int nb0, int nb1, int nb2, const uint8_t* act_in, uint8_t* act_out,
+                           int nb0, int nb1, int nb2, uint8_t* act_in, uint8_t* act_out,
                            int* any_marked, hipStream_t s);
 hipError_t launch_ca_finalize(bool is_int, const void* dist, double* act, int64_t n, hipStream_t s);
 
