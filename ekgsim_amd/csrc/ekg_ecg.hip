@@ -1925,7 +1925,8 @@ hipError_t launch_ecg_chunk(const GroupArgs& a, hipStream_t s)
 
 hipError_t launch_class_boxes(const GroupArgs& a, const ClassLaunch& c, hipStream_t s)
 {
-    if (c.blocks < 1 || c.blocks > 0x7fffffffLL || c.n_segs < 1) return hipErrorInvalidValue;
+    if (c.blocks < 0 || c.blocks > 0x7fffffffLL || c.n_segs < 1) return hipErrorInvalidValue;
+    if (c.blocks == 0) return hipSuccess;  // hearts without class cells: their sums are zero
     hipLaunchKernelGGL(ecg_class_box_kernel, dim3((unsigned)c.blocks), dim3(64 * CB_WAVES), 0, s, a.hearts,
                        a.segs + c.seg0, c.n_segs, a.rowpos, a.lead_pos, a.gsum);
     return hipGetLastError();

@@ -906,7 +906,7 @@ size_t group_device_bytes(const GroupPlan& g)
         if (g.mfma && fits && L.n_classes > 0) {
             // lines of class sums (before the cells are built: each class in
             // an eighth of the regions)
-            const int64_t lines = L.cells_built[g.nhood] ? L.n_lines[g.nhood] : (int64_t)8 * L.n_classes;
+            const int64_t lines = L.cells_built[g.nhood] ? std::max(1, L.n_lines[g.nhood]) : (int64_t)8 * L.n_classes;
             gsum += lines * r.L * 8;
             line_max = std::max(line_max, lines);
         }
@@ -1078,8 +1078,10 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         for (int r = 0; r < B; ++r) {
             const EcgLayout& hl = g.reqs[r].h->layout;
             if (hl.n_classes == 0) continue;
-            need_lines += (int64_t)g.reqs[r].L * hl.n_lines[g.nhood] / 16 + hl.n_lines[g.nhood];
-            one_row = std::max<int64_t>(one_row, hl.n_lines[g.nhood]);
+            // (a heart that is one class as a whole has no lines: its cells cancel)
+            const int64_t lines = std::max(1, hl.n_lines[g.nhood]);
+            need_lines += g.reqs[r].L * lines / 16 + lines;
+            one_row = std::max(one_row, lines);
             fixed += fixed_class_bytes(g.reqs[r], LP);
         }
         const int64_t cap = std::max(one_row, ws.arena ? fixed / LINE_BYTES : std::min(need_lines, GSUM_BYTES / LINE_BYTES));
