@@ -1645,7 +1645,7 @@ __global__ __launch_bounds__(256) void class_sums_kernel(
     const double* g = gsum + (sg.goff + (int64_t)(rg - sg.rg0) * H.n_lines) * 16 + (t & 15);
     double s = 0.0;
     const int q1 = H.cs_off[k + 1];
-#pragma unroll 4
+#pragma unroll 8
     for (int q = H.cs_off[k]; q < q1; ++q) s += g[(int64_t)16 * H.cs_line[q]];
     const ReqDev& R = reqs[row >> 5];
     const int i = row & 31, l = H.classes[k].x;
@@ -1670,11 +1670,18 @@ __global__ __launch_bounds__(256) void class_sums_kernel(
 // terms factor through its sums.  Samples from Tn on receive nothing, as in
 // the reduction.  One block of CL_WAVES waves per (request, 64 steps), one
 // step per lane: wave w adds the classes [w n / CL_WAVES, (w+1) n / CL_WAVES)
-// in order, two FMAs per lead, then the waves' sums are added in wave order.
-// The time-independent sum over the classes of k0 sum G (csums holds k0 sum G)
-// is formed once per block: thread (part p, lead i) adds classes p, p + NP,
-// ..., then lead i's parts are added in order.
-constexpr int CL_WAVES = 4;
+// in order, two FMAs per lead, then the waves' sums are added in a fixed
+// order.  The time-independent sum over the classes of k0 sum G (csums holds
+// k0 sum G) is formed once per block: thread (part p, lead i) adds classes p,
+// p + NP, ..., then lead i's parts are added in order.
+//
+// With few requests the chain of a wave's classes bounds it, one trip for a
+// class's sums after the other; hence eight waves (few classes each) and the
+// sums' cache lines brought into L2 at the start, all at once.  One 12-lead
+// request, 170 classes, 800 steps: 26.5 us with four waves and no such loads,
+// 12.6 us now; two leads, 241 classes: 18.6 -> 13.1 us.  With many requests
+// the FMAs bound it: 256 requests 64 us both ways.
+constexpr int CL_WAVES = 8;
 
 template <int LP>
 __global__ __launch_bounds__(64 * CL_WAVES) void ecg_class_kernel(
@@ -1684,7 +1691,8 @@ __global__ __launch_bounds__(64 * CL_WAVES) void ecg_class_kernel(
     double* __restrict__ ecg)
 {
     constexpr int NP = 64 * CL_WAVES / LP;  // parts of the k0 sum per lead
-    __shared__ double s_acc[CL_WAVES - 1][LP][64];
+    constexpr int HW = CL_WAVES / 2;
+    __shared__ double s_acc[HW][LP][64];
     __shared__ double s_k0[NP][LP];
     // Blocks go round-robin over the 8 XCDs.  With cl_per_req blocks for
     // every request and B a multiple of 8, XCD x takes requests x, x + 8, ...
@@ -1705,8 +1713,22 @@ __global__ __launch_bounds__(64 * CL_WAVES) void ecg_class_kernel(
     const int j0 = jb * 64;
     if (j0 >= R.Tn) return;  // the whole block
     const int j = j0 + lane;
-    const bool live = j < R.Tn;
     const double t = tgrid[R.t_off + j];  // j < Tp: in the grid
+    // One load per 128-byte line of the request's sums and the class records
+    // brings them into this XCD's L2 together: the scalar loads below come one
+    // class after the other, each as long as a trip to memory otherwise.
+    int line = 0;
+    {
+        const char* const b0 = (const char*)(csums + R.cls_off * 3 * LP);
+        const char* const b1 = (const char*)H.classes;
+        const char* const b2 = (const char*)H.class_a;
+        const int n0 = H.n_classes * 3 * LP * 8, n1 = H.n_classes * 16, n2 = H.n_classes * 8;
+        for (int o = 128 * (int)threadIdx.x; o < n0; o += 128 * 64 * CL_WAVES) {
+            line ^= *(const int*)(b0 + o);
+            if (o < n1) line ^= *(const int*)(b1 + o);
+            if (o < n2) line ^= *(const int*)(b2 + o);
+        }
+    }
     if ((int)threadIdx.x < NP * LP) {
         const int p = (int)threadIdx.x / LP, i = (int)threadIdx.x - p * LP;
         double c = 0.0;
@@ -1714,6 +1736,7 @@ __global__ __launch_bounds__(64 * CL_WAVES) void ecg_class_kernel(
         for (int k = p; k < H.n_classes; k += NP) c += csums[(R.cls_off + k) * 3 * LP + i];
         s_k0[p][i] = c;
     }
+    asm volatile("" ::"v"(line));  // the loads stand
     double acc[LP];
 #pragma unroll
     for (int i = 0; i < LP; ++i) acc[i] = 0.0;
@@ -1744,20 +1767,25 @@ __global__ __launch_bounds__(64 * CL_WAVES) void ecg_class_kernel(
 #pragma unroll
         for (int i = 0; i < LP; ++i) acc[i] = __builtin_fma(SY, cs[2 * LP + i], __builtin_fma(SX, cs[LP + i], acc[i]));
     }
-    if (w > 0)
+    // the upper waves' sums onto the lower ones', then one thread per (lead,
+    // step) adds the lower waves in order
+    if (w >= HW)
 #pragma unroll
-        for (int i = 0; i < LP; ++i) s_acc[w - 1][i][lane] = acc[i];
+        for (int i = 0; i < LP; ++i) s_acc[w - HW][i][lane] = acc[i];
     __syncthreads();
-    if (w == 0 && live) {
+    if (w < HW)
 #pragma unroll
-        for (int i = 0; i < LP; ++i) {
-            double v = acc[i];
+        for (int i = 0; i < LP; ++i) s_acc[w][i][lane] += acc[i];
+    __syncthreads();
+    for (int q = threadIdx.x; q < R.L * 64; q += 64 * CL_WAVES) {
+        const int i = q >> 6;
+        if (j0 + lane >= R.Tn) continue;
+        double v = s_acc[0][i][lane], c0 = 0.0;
 #pragma unroll
-            for (int ww = 0; ww < CL_WAVES - 1; ++ww) v += s_acc[ww][i][lane];
-            double c0 = 0.0;
-            for (int p = 0; p < NP; ++p) c0 += s_k0[p][i];
-            if (i < R.L) ecg[R.ecg_off + (int64_t)i * R.T + j] += v + c0;
-        }
+        for (int ww = 1; ww < HW; ++ww) v += s_acc[ww][i][lane];
+#pragma unroll 8
+        for (int p = 0; p < NP; ++p) c0 += s_k0[p][i];
+        ecg[R.ecg_off + (int64_t)i * R.T + j] += v + c0;
     }
 }
 
