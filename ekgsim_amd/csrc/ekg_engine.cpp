@@ -1164,15 +1164,15 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         ws.h_grids.swap(grid_bytes);
     }
     if (!dev_in) {
+        // coefficients and positions in one upload: each is about 10 us of host
+        // and copy engine before the group's first kernel
+        const size_t nk = ws.h_k.size();
+        ws.h_k.insert(ws.h_k.end(), ws.h_pos.begin(), ws.h_pos.end());
         ws.need(ws.layer_k, ws.h_k.size() * 8);
-        ws.need(ws.lead_pos, ws.h_pos.size() * 8);
         hip_check(hipMemcpyAsync(ws.layer_k.p, ws.h_k.data(), ws.h_k.size() * 8, hipMemcpyHostToDevice, stream),
-                  "upload AP coefficients");
-        hip_check(hipMemcpyAsync(ws.lead_pos.p, ws.h_pos.data(), ws.h_pos.size() * 8, hipMemcpyHostToDevice,
-                                 stream),
-                  "upload lead positions");
+                  "upload AP coefficients and lead positions");
         d_k = ws.layer_k.as<double>();
-        d_pos = ws.lead_pos.as<double>();
+        d_pos = d_k + nk;
     }
     const char* tb = static_cast<const char*>(ws.hearts.p);
     const int64_t* stp = reinterpret_cast<const int64_t*>(tb + o_st);

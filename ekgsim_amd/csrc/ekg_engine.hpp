@@ -41,7 +41,7 @@ struct DevBuf {
 
 // Device workspace of one launch group on one stream (grow-only buffers).
 struct Workspace {
-    DevBuf hearts, reqs, starts, layer_k, lead_pos, tgrid, thl, lc, xy, G, aux, sums, bnd, pre_rng,
+    DevBuf hearts, reqs, starts, layer_k, tgrid, thl, lc, xy, G, aux, sums, bnd, pre_rng,
         pre_ab, partial, gsum, csums, ecg;
     std::vector<double> h_k, h_pos, h_tgrid;
     std::vector<float> h_thl;
