@@ -69,13 +69,15 @@ def lead_field_cells(layer):
     return int(cnt[myo].sum())
 
 
-# Algorithmic work, counted per unit.  Class-window kernel (the dominant one
+# Algorithmic work, counted per unit.  Class-box kernel (the dominant one
 # when the heart has activation classes):
-#   per (class-window entry, lead): 8 FP64 matrix-core flops (|e|^2 as a
-#     4-term product, 4 FMAs) and 3 FP32 flops (rsq 1, |e|^-3 2), the lead
-#     weight shared by the entry's classes;
-#   per (class cell, lead): 8 FP64 matrix-core flops (an FMA for each of the
-#     coefficients D0, D1, D2, K).
+#   per (myocardial cell, lead): 1 FP64 flop (|e|^2 as the sum of a row's and a
+#     column's part) and 3 FP32 flops (rsq 1, |e|^-3 2), the lead weight
+#     shared by the cell's classes;
+#   per (class cell, lead): 8 flops (a multiply-add for each of the
+#     coefficients D0, D1, D2, K).  The kernel does these exactly, in integers
+#     on the int8 matrix cores (four 8-bit limbs of a weight), so the rate
+#     below is that of the equivalent FP64 work, not of a pipe.
 # Chunk kernel (dominant without classes):
 #   per lead-weight evaluation (voxel, lead, cell): 6 FP64 flops (|e|^2 as
 #     one FMA from the voxel's own |e|^2 and the dipole sum, the dipole
@@ -85,7 +87,7 @@ def lead_field_cells(layer):
 # Both count at full weight against 78.6 TFLOP/s: the build disables packed
 # FP32, so an FP32 vector operation issues at the FP64 vector rate, which on
 # MI355X equals the FP64 matrix rate.
-FP32_PER_CLASS_ENTRY, FP64_PER_CLASS_ENTRY, FP64_PER_CLASS_CELL = 3, 8, 8
+FP32_PER_CLASS_WEIGHT, FP64_PER_CLASS_WEIGHT, FP64_PER_CLASS_CELL = 3, 1, 8
 FP32_PER_CELL, FP64_PER_CELL = 3, 6
 FP32_PER_WINDOW_STEP = 11
 # Serving bursts: warm-up bursts before the measured ones, and measured bursts
@@ -98,17 +100,17 @@ NAIVE_LANE_CYCLES, LANE_PEAK = 38, 256 * 64 * 2.4e9
 # HBM bytes per launch of the dominant kernel on this workload, from
 # rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE, each scaled by its reading for a
 # 256 MiB calibration copy: with activation classes
-# (profiles/ecg_class_window_kernel_128cubed_batch256_hbm_traffic.md) and
+# (profiles/ecg_class_box_kernel_128cubed_batch256_hbm_traffic.md) and
 # without (profiles/ecg_chunk_kernel_128cubed_batch256_hbm_traffic.md).
-TRAFFIC_BYTES = {"ecg_class_window_kernel": 436566943, "ecg_chunk_kernel": 1131874216}
+TRAFFIC_BYTES = {"ecg_class_box_kernel": 436566943, "ecg_chunk_kernel": 1131874216}
 # Issue-pipe occupancy of the dominant kernel on this workload, from one
 # rocprofv3 --pmc pass (SQ_VALU_MFMA_BUSY_CYCLES, SQ_INSTS_VALU minus the MFMA
 # instructions at 4 cycles each, SQ_VALU_MFMA_COEXEC_CYCLES, GRBM_GUI_ACTIVE)
-# over 1024 SIMDs: profiles/ecg_class_window_kernel_128cubed_batch256_pipes.md
+# over 1024 SIMDs: profiles/ecg_class_box_kernel_128cubed_batch256_pipes.md
 # and profiles/ecg_chunk_kernel_128cubed_batch256_pipes.md.  The matrix cores
 # and the vector ALU never overlap (COEXEC 0), so their sum is the fraction of
 # the kernel's cycles spent issuing.
-PIPES = {"ecg_class_window_kernel": {"mfma_busy": 0.563, "valu_issue": 0.294, "coexec": 0.0},
+PIPES = {"ecg_class_box_kernel": {"mfma_busy": 0.563, "valu_issue": 0.294, "coexec": 0.0},
          "ecg_chunk_kernel": {"mfma_busy": 0.116, "valu_issue": 0.806, "coexec": 0.0}}
 
 
@@ -470,15 +472,15 @@ def main():
     act_myo = act_grid[h.layer > 0]
     info = heart.layout_info("3D4") if args.kernel != "valu" else None
     n_classes = info["classes"] if info and heart.get_tune()["class_min"] >= 0 else 0
-    win = cells = ccells = centries = 0
+    win = cells = ccells = cweights = 0
     if n_classes > 0:
-        # the class-window kernel: every entry's weight and every class cell's
+        # the class-box kernel: every cell's weight and every class cell's
         # contraction once per (request, lead)
-        dom = "ecg_class_window_kernel"
+        dom = "ecg_class_box_kernel"
         ccells = B * L * info["class_cells"]
-        centries = B * L * info["class_entries"]
-        f64 = FP64_PER_CLASS_CELL * ccells + FP64_PER_CLASS_ENTRY * centries
-        f32 = FP32_PER_CLASS_ENTRY * centries
+        cweights = B * L * V
+        f64 = FP64_PER_CLASS_CELL * ccells + FP64_PER_CLASS_WEIGHT * cweights
+        f32 = FP32_PER_CLASS_WEIGHT * cweights
     else:
         dom = "ecg_chunk_kernel" if args.kernel != "valu" else "ecg_fused_kernel"
         win = sum(window_voxel_steps(act_myo, float(k[0][1]), 0.0, 1.0, T) for k in ks)
@@ -735,10 +737,10 @@ def main():
             "fp64_flops_per_launch": f64,
             "fp32_flops_per_launch": f32,
             "class_cell_leads_per_launch": ccells,
-            "class_entry_leads_per_launch": centries,
+            "class_weight_leads_per_launch": cweights,
             "lead_weight_evaluations_per_launch": cells,
             "window_voxel_steps_per_launch": win,
-            "per_unit": {"class_entry_lead": {"fp32": FP32_PER_CLASS_ENTRY, "fp64": FP64_PER_CLASS_ENTRY},
+            "per_unit": {"class_weight_lead": {"fp32": FP32_PER_CLASS_WEIGHT, "fp64": FP64_PER_CLASS_WEIGHT},
                          "class_cell_lead": {"fp32": 0, "fp64": FP64_PER_CLASS_CELL},
                          "lead_weight_evaluation": {"fp32": FP32_PER_CELL, "fp64": FP64_PER_CELL},
                          "window_voxel_step": {"fp32": FP32_PER_WINDOW_STEP, "fp64": 2 * L},

@@ -14,6 +14,11 @@
 //   chunk_sums    per (request, chunk): sum G, sum G P', sum G Q' in FP64
 //                 and the chunk's tile bounds [z, f): before z every voxel
 //                 is far before its upstroke, from f on every sigmoid is 1
+//   ecg_chunk     per (request, chunk), the matrix-core path: the two above and
+//                 ecg_fused in one kernel, the lead weights kept on chip
+//   ecg_class_box per (region of class cells, row of 16 leads): each cell's lead
+//                 weight once, contracted into its classes' sums on the int8
+//                 matrix cores; class_sums adds a class's regions
 //   layer_prefix  per (request, layer, tile): prefix sums of the saturated
 //                 chunks and the range of chunks still in transition
 //   ecg_fused     per (request, chunk), transition tiles only: AP
@@ -21,6 +26,7 @@
 //                 accumulation on the matrix cores or the vector ALUs)
 //   ecg_reduce    per (request, lead, step): closed form of the saturated
 //                 chunks + fixed-order FP64 sum of the transition partials
+//   ecg_class     per (request, 64 steps): adds the activation classes
 //
 // Every launch is checked on the host against the buffer extents it assumes
 // (ekg_engine.cpp) before it is issued.
@@ -741,7 +747,7 @@ constexpr int CH_LEADS = 2;   // leads per pass of the chunk kernel's lead field
 // sigma = e(u) . d, which the dipole product needs anyway:
 //   e(u+d) . d = sigma - |d|^2,   |e(u+d)|^2 = |e(u)|^2 + |d|^2 - 2 sigma,
 // one FMA per cell.  The FP64 value differs from the cell's directly summed
-// |e|^2 (its own evaluation, or the class-window kernel's matrix product) by a few
+// |e|^2 (its own evaluation, or the class-box kernel's separable sum) by a few
 // 1e-16 relative, so after rounding to FP32 a cell gets the same weight from
 // every voxel that evaluates it except where those FP64 values straddle an
 // FP32 rounding boundary (about one in 1e8 evaluations, each a one-ulp weight

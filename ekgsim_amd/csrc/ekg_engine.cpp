@@ -254,7 +254,7 @@ constexpr double CHUNK_SPAN_MS = 16.0;
 // one layer with one activation time takes the class path.
 constexpr int DEFAULT_CLASS_MIN = 64;
 // Largest class chunk (voxels): a class is kept as a run of class chunks
-// (layout bookkeeping; the class-window kernel takes whole classes).
+// (layout bookkeeping; the class-box kernel takes whole classes).
 constexpr int64_t CLASS_CHUNK = 4096;
 // Windows of six classes and pieces of 1024 groups of 16 window entries: the
 // units in which layout_info states a layout's size, and the fixed workspace
@@ -1275,18 +1275,19 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
             // `stream`, beside the AP tables, chunk, prefix and reduction
             // kernels on the side stream (they share no buffer); the
             // class ECG kernel adds to the reduction's output after both.
-            // The branch with more of the voxels is launched first, but for
-            // the AP tables, whose time on the device covers the first
-            // class launches' on the host.  One 12-lead request on a 128^3
-            // heart, classes mostly: 167 us with the side branch first, 142
-            // after the AP tables, 126 ahead of all; 128 requests on a
-            // 24-layer heart, classes few: 578, 575, 582 us.
+            // The branch with more of the voxels is launched first; a small
+            // class branch goes out while the chunk kernel runs.  One 12-lead
+            // request on a 128^3 heart, classes mostly: 167 us with the whole side
+            // branch first, 142 after the AP tables, 126 ahead of all.
+            // One on a 24-layer heart, classes few: 124 us with the side branch
+            // first, 121 after the AP tables, 114 after the chunk
+            // kernel; 128 such requests 578, 573, 573, and 582 us ahead of all.
             hip_check(hipEventRecord(ws.ev_fork, stream), "hipEventRecord");
             if (classes_lead) classes();
             hip_check(hipStreamWaitEvent(ws.side, ws.ev_fork, 0), "hipStreamWaitEvent");
             hip_check(ekgk::launch_ap_tables(a, ws.side), "ap_tables launch");
-            if (!classes_lead) classes();
             hip_check(ekgk::launch_ecg_chunk(a, ws.side), "ecg_chunk launch");
+            if (!classes_lead) classes();
             hip_check(ekgk::launch_layer_prefix(a, ws.side), "layer_prefix launch");
             hip_check(ekgk::launch_ecg_reduce(a, ws.side), "ecg_reduce launch");
             hip_check(hipEventRecord(ws.ev_join, ws.side), "hipEventRecord");

@@ -51,7 +51,7 @@ struct Workspace {
     hipGraphExec_t graph = nullptr;
     std::vector<char> graph_key;
     // second stream of a group's launches (the chunk, prefix and reduction
-    // kernels beside the class-window kernel) and its fork and join events;
+    // kernels beside the class-box kernel) and its fork and join events;
     // created by ensure_side, on the device that is current
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
