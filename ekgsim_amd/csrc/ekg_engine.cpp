@@ -889,12 +889,37 @@ void append(std::vector<char>& buf, const T* p, size_t n)
     buf.insert(buf.end(), c, c + n * sizeof(T));
 }
 
+// Lines of a group's class sums, and the most of one row: the leads of each run
+// of consecutive requests of one heart fill rows of 16, a row has a line per
+// (region, class) of the heart.  Before the cells are built, each class counts in an
+// eighth of the regions; a heart that is one class as a whole (no lines: its
+// cells cancel) counts one.
+struct ClassLines {
+    int64_t all = 0, row = 0;
+};
+
+ClassLines class_lines(const GroupPlan& g)
+{
+    ClassLines c;
+    for (size_t r = 0; r < g.reqs.size();) {
+        const Heart* h = g.reqs[r].h;
+        const EcgLayout& L = h->layout;
+        int64_t leads = 0;
+        for (; r < g.reqs.size() && g.reqs[r].h == h; ++r) leads += g.reqs[r].L;
+        // a layout for the other path is sized as one without classes
+        if (!(g.mfma && L.valid && L.n_classes > 0)) continue;
+        const int64_t lines = L.cells_built[g.nhood] ? std::max(1, L.n_lines[g.nhood]) : (int64_t)8 * L.n_classes;
+        c.all += (leads + 15) / 16 * lines;
+        c.row = std::max(c.row, lines);
+    }
+    return c;
+}
+
 }  // namespace
 
 size_t group_device_bytes(const GroupPlan& g)
 {
     size_t s = 0;
-    int64_t gsum = 0, line_max = 0;
     const int LP = g.LP;
     for (const ReqSpec& r : g.reqs) {
         const EcgLayout& L = r.h->layout;
@@ -903,13 +928,6 @@ size_t group_device_bytes(const GroupPlan& g)
         const bool fits = L.valid && (L.class_min == 0 || g.mfma);
         const int64_t est = std::max<int64_t>(1, V / 64 + r.h->max_layer + 4);
         const int64_t nmix = fits ? L.n_chunks : est;
-        if (g.mfma && fits && L.n_classes > 0) {
-            // lines of class sums (before the cells are built: each class in
-            // an eighth of the regions)
-            const int64_t lines = L.cells_built[g.nhood] ? std::max(1, L.n_lines[g.nhood]) : (int64_t)8 * L.n_classes;
-            gsum += lines * r.L * 8;
-            line_max = std::max(line_max, lines);
-        }
         const int64_t ncls = fits ? L.n_classes : 0;
         const int64_t rows = g.mfma ? 0 : V + ekgk::MFMA_PAD;
         s += (size_t)r.nl * 9 * 8 + (size_t)r.L * 3 * 8 + (size_t)r.Tp * 16;
@@ -923,7 +941,8 @@ size_t group_device_bytes(const GroupPlan& g)
         // record, heart, seven start tables, class rows
         s += sizeof(ekgk::ReqDev) + sizeof(ekgk::HeartDev) + 7 * 8 + sizeof(ekgk::ClassSeg) + r.L * 12;
     }
-    return s + (size_t)std::max(line_max * LINE_BYTES, std::min(gsum + line_max * LINE_BYTES, GSUM_BYTES));
+    const ClassLines c = class_lines(g);
+    return s + (size_t)std::max(c.row * LINE_BYTES, std::min(c.all * LINE_BYTES, GSUM_BYTES));
 }
 
 void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, const double* d_k,
@@ -1074,17 +1093,10 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     std::vector<ekgk::ClassLaunch> launches;
     std::vector<int> rowtab, rowpos, rgseg;
     if (g.mfma && st_cs[B] > 0) {
-        int64_t need_lines = 0, one_row = 0, fixed = 0;
-        for (int r = 0; r < B; ++r) {
-            const EcgLayout& hl = g.reqs[r].h->layout;
-            if (hl.n_classes == 0) continue;
-            // (a heart that is one class as a whole has no lines: its cells cancel)
-            const int64_t lines = std::max(1, hl.n_lines[g.nhood]);
-            need_lines += g.reqs[r].L * lines / 16 + lines;
-            one_row = std::max(one_row, lines);
-            fixed += fixed_class_bytes(g.reqs[r], LP);
-        }
-        const int64_t cap = std::max(one_row, ws.arena ? fixed / LINE_BYTES : std::min(need_lines, GSUM_BYTES / LINE_BYTES));
+        const ClassLines cl = class_lines(g);
+        int64_t fixed = 0;
+        for (const ReqSpec& r : g.reqs) fixed += fixed_class_bytes(r, LP);
+        const int64_t cap = std::max(cl.row, ws.arena ? fixed / LINE_BYTES : std::min(cl.all, GSUM_BYTES / LINE_BYTES));
         ws.need(ws.gsum, (size_t)(cap * LINE_BYTES));
         int64_t block0 = 0, used = cap;  // lines taken in the current launch
         for (int r = 0; r < B;) {
