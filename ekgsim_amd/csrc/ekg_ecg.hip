@@ -1534,7 +1534,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                     // the nearest cell itself, in FP64
                     const double rz = fmin(fmax(rint(qz), 0.0), 3.0), ry = fmin(fmax(rint(qy), 0.0), 7.0),
                                  rx = fmin(fmax(rint(qx), 0.0), 7.0);
-                    const double d2 = fmax((qz - rz) * (qz - rz) + (qy - ry) * (qy - ry) + (qx - rx) * (qx - rx), 0x1p-84);
+                    const double d2 = fmax((qz - rz) * (qz - rz) + (qy - ry) * (qy - ry) + (qx - rx) * (qx - rx), 0x1p-86);
                     m = ((int)((__double_as_longlong(d2) >> 52) & 2047) - 1023 + 20) >> 1;
                     // passes of 30 bits until the smallest weight's 24 bits are
                     // covered: log2 s >= -1.5 (floor(log2 |e|^2) + 1)
@@ -1542,6 +1542,9 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                     np = 1 + (23 + ((3 * ef + 1) >> 1) + 29) / 30;
                 }
             }
+            // From 2^-42.67 voxels on (|e|^2 at most 2^-85.33, m at its least, -33) the
+            // FP32 weight is infinite: scaled by 2^(3 m), 2^29 or more.
+            const float s_inf = m <= -33 ? 0x1p29f : __builtin_inff();
             const double st = __longlong_as_double((long long)(1023 - m) << 52);  // 2^-m
             double sc = __longlong_as_double((long long)(1023 - 3 * m) << 52);
             for (int pass = 0;; ++pass) {
@@ -1589,9 +1592,10 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                             s[x] = r * r * r;
                         }
                         if (hot) {
-                            // an electrode on the centre of a cell with dipoles: its sums are not finite
+                            // an electrode on the centre of a cell with dipoles, or too near for a
+                            // finite FP32 weight: its sums are not finite
 #pragma unroll
-                            for (int x = 0; x < 4; ++x) bad |= ((cm >> (4 * y + x)) & 1u) && s[x] == __builtin_inff();
+                            for (int x = 0; x < 4; ++x) bad |= ((cm >> (4 * y + x)) & 1u) && s[x] >= s_inf;
 #pragma unroll 1
                             for (int h = 0; h < pass; ++h)
 #pragma unroll
