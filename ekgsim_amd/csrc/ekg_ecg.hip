@@ -1525,7 +1525,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
             npk = pkt[(int64_t)64 * bn];
             nin = ini[(int64_t)64 * bn];
             int np = 1;
-            bool hot = false;
+            bool hot = false, bad = false;
             if (per_box) {
                 const ScaleRange br = scale_range((float)qz, (float)qy, (float)qx, 1.5f, 3.5f, 3.5f);
                 m = br.m;
@@ -1534,7 +1534,16 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                     // the nearest cell itself, in FP64
                     const double rz = fmin(fmax(rint(qz), 0.0), 3.0), ry = fmin(fmax(rint(qy), 0.0), 7.0),
                                  rx = fmin(fmax(rint(qx), 0.0), 7.0);
-                    const double d2 = fmax((qz - rz) * (qz - rz) + (qy - ry) * (qy - ry) + (qx - rx) * (qx - rx), 0x1p-86);
+                    const double dc = (qz - rz) * (qz - rz) + (qy - ry) * (qy - ry) + (qx - rx) * (qx - rx);
+                    // On the centre of a cell with dipoles, or so near it (1.44e-13 voxels) that
+                    // the FP32 weight overflows, the lead's sums are not finite.
+                    const float r = __builtin_amdgcn_rsqf((float)dc);
+                    if (r * r * r == __builtin_inff()) {
+                        const int iz = (int)rz, iy = (int)ry, ix = (int)rx;
+                        const uint64_t cm = H.cmask[4 * b + 2 * (iy >> 2) + (ix >> 2)];
+                        bad = (cm >> (16 * iz + 4 * (iy & 3) + (ix & 3))) & 1;
+                    }
+                    const double d2 = fmax(dc, 0x1p-86);
                     m = ((int)((__double_as_longlong(d2) >> 52) & 2047) - 1023 + 20) >> 1;
                     // passes of 30 bits until the smallest weight's 24 bits are
                     // covered: log2 s >= -1.5 (floor(log2 |e|^2) + 1)
@@ -1542,11 +1551,8 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                     np = 1 + (23 + ((3 * ef + 1) >> 1) + 29) / 30;
                 }
             }
-            // From 2^-42.67 voxels on (|e|^2 at most 2^-85.33, m at its least, -33) the
-            // FP32 weight is infinite: scaled by 2^(3 m), 2^29 or more.
-            const float s_inf = m <= -33 ? 0x1p29f : __builtin_inff();
             const double st = __longlong_as_double((long long)(1023 - m) << 52);  // 2^-m
-            double sc = __longlong_as_double((long long)(1023 - 3 * m) << 52);
+            double sc = bad ? __builtin_nan("") : __longlong_as_double((long long)(1023 - 3 * m) << 52);
             for (int pass = 0;; ++pass) {
                 // |e|^2 x 4^-m = X[x] + Y[y], formed in each pass (the pin keeps them
                 // out of the registers of the tile loop below)
@@ -1577,11 +1583,9 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                     }
                 };
                 load_tile();
-                bool bad = false;
                 i32x4 W[4][4];  // [sub-brick][limb]: bytes 4 y + x
 #pragma unroll
                 for (int sb = 0; sb < 4; ++sb) {
-                    const unsigned cm = hot ? (unsigned)(H.cmask[4 * b + sb] >> (16 * zq)) : 0u;
 #pragma unroll
                     for (int y = 0; y < 4; ++y) {
                         if (!((rows >> (4 * sb + y)) & 1)) continue;
@@ -1592,10 +1596,6 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                             s[x] = r * r * r;
                         }
                         if (hot) {
-                            // an electrode on the centre of a cell with dipoles, or too near for a
-                            // finite FP32 weight: its sums are not finite
-#pragma unroll
-                            for (int x = 0; x < 4; ++x) bad |= ((cm >> (4 * y + x)) & 1u) && s[x] >= s_inf;
 #pragma unroll 1
                             for (int h = 0; h < pass; ++h)
 #pragma unroll
@@ -1607,10 +1607,6 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
 #pragma unroll
                         for (int j = 0; j < 4; ++j) W[sb][j][y] = o4[j];
                     }
-                }
-                if (hot) {
-                    const int any4 = (int)bad | __shfl_xor((int)bad, 16, 64);
-                    if (any4 | __shfl_xor(any4, 32, 64)) sc = __builtin_nan("");
                 }
                 const double cz = qz * sc, cy = qy * sc, cx = qx * sc;
                 for (;;) {
