@@ -1408,6 +1408,15 @@ __device__ __forceinline__ void limbs4(const int q[4], int out[4])
     out[3] = (int)(__builtin_amdgcn_perm(d, b, 0x07060302u) ^ 0x80808080u);
 }
 
+// Orders a wave's LDS accesses before it ahead of those after it, where one lane
+// reads what another wrote: for the compiler; the LDS serves a wave in order.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // FP32 to int32 toward zero, saturating, NaN to 0 (the instruction's own rule).
 __device__ __forceinline__ int cvt_i32(float x)
 {
@@ -1515,7 +1524,9 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
         }
         for (int b = b0; b < reg.y; b += CB_WAVES) {
             const i32x4 tr = npk;  // lane l < 16: tile l {sub-bricks, 4 slot bytes, first block, 0}
+            wave_lds_fence();      // the box before: its reads of s_init and its sums in s_acc
             s_init[w][lane] = nin;
+            wave_lds_fence();
             // lane 16: {tiles, rows (4 sub-brick + y) in use, 0, 0}; lane 17: first cell + 1
             const int nt = __builtin_amdgcn_readlane(tr.x, 16), rows = __builtin_amdgcn_readlane(tr.y, 16);
             // electrode relative to the box's first cell
@@ -1588,7 +1599,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                 for (int sb = 0; sb < 4; ++sb) {
 #pragma unroll
                     for (int y = 0; y < 4; ++y) {
-                        if (!((rows >> (4 * sb + y)) & 1)) continue;
+                        if (!((rows >> (4 * sb + y)) & 1)) continue;  // only zero coefficients
                         float s[4];
 #pragma unroll
                         for (int x = 0; x < 4; ++x) {
@@ -1608,6 +1619,9 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                         for (int j = 0; j < 4; ++j) W[sb][j][y] = o4[j];
                     }
                 }
+                // rows left out: whatever their registers hold, it counts as a value
+#pragma unroll
+                for (int i = 0; i < 16; ++i) asm("" : "+v"((&W[0][0])[i]));
                 const double cz = qz * sc, cy = qy * sc, cx = qx * sc;
                 for (;;) {
                     const i32x4 c0 = s_init[w][4 * (ti & 15) + zq];
