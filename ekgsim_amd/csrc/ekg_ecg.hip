@@ -1761,8 +1761,8 @@ __global__ __launch_bounds__(64 * CL_WAVES) void ecg_class_kernel(
         const char* const b0 = (const char*)(csums + R.cls_off * 3 * LP);
         const char* const b1 = (const char*)H.classes;
         const char* const b2 = (const char*)H.class_a;
-        const int n0 = H.n_classes * 3 * LP * 8, n1 = H.n_classes * 16, n2 = H.n_classes * 8;
-        for (int o = 128 * (int)threadIdx.x; o < n0; o += 128 * 64 * CL_WAVES) {
+        const int64_t n = H.n_classes, n0 = n * 3 * LP * 8, n1 = n * 16, n2 = n * 8;
+        for (int64_t o = 128 * (int)threadIdx.x; o < n0; o += 128 * 64 * CL_WAVES) {
             line ^= *(const int*)(b0 + o);
             if (o < n1) line ^= *(const int*)(b1 + o);
             if (o < n2) line ^= *(const int*)(b2 + o);
