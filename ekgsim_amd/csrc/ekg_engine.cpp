@@ -1060,8 +1060,12 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         // Long ranges of chunks in transition: a heart of many chunks, from before
         // its last activation on (a request that starts later meets every
         // chunk saturated).  512 chunks put about 170 into a range of the upstroke,
-        // where the sums in parts begin to pay (48^3: 157 chunks, 12 us either way).
-        const bool parts = h.layout.n_chunks >= LONG_RANGES && q.start < h.layout.a_last;
+        // where the sums in parts begin to pay (48^3: 157 chunks, 12 us either way;
+        // one 12-lead request on the 80^3, 96^3 and 128^3 conduction-matrix hearts
+        // 104, 98 and 137 us, 140, 152 and 224 without).  On the vector-ALU path a
+        // tile has 64 steps, so that from 8 leads on its sums fill a block without
+        // parts: 12 leads on 128^3 404 us, 510 in parts; 2 leads 338 and 226.
+        const bool parts = (g.mfma || LP == 4) && h.layout.n_chunks >= LONG_RANGES && q.start < h.layout.a_last;
         st_red[r + 1] = st_red[r] + (parts ? 0 : (q.L * tiles) << R.bt_shift);
         st_redp[r + 1] = st_redp[r] + (parts ? tiles : 0);
         st_cs[r + 1] = st_cs[r] + z.classes;
