@@ -117,7 +117,7 @@ void Ctx::collect_timings()
         float ms = 0.f;
         hip_check(hipEventElapsedTime(&ms, pr.first, pr.second), "hipEventElapsedTime");
         fused_ms += ms;
-        ++fused_launches;
+        fused_launches += pr.counts;
         free_events.push_back(pr.first);
         free_events.push_back(pr.second);
     }
@@ -1267,6 +1267,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         // kernel, or without classes the chunk kernel (matrix-core path), or
         // the fused transition-tile kernel (vector ALUs).
         hipEvent_t e0 = nullptr, e1 = nullptr;
+        bool counts = true;
         auto tic = [&]() {
             if (!timed) return;
             e0 = ctx.get_event();
@@ -1276,13 +1277,14 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         auto toc = [&]() {
             if (!timed) return;
             hip_check(hipEventRecord(e1, stream), "hipEventRecord");
-            ctx.pending.emplace_back(e0, e1);
+            ctx.pending.push_back({e0, e1, counts});
+            counts = false;
         };
         auto classes = [&]() {
             for (const ekgk::ClassLaunch& c : launches) {
-                if (&c == &launches[0]) tic();
+                tic();
                 hip_check(ekgk::launch_class_boxes(a, c, stream), "class_box launch");
-                if (&c == &launches[0]) toc();
+                toc();
                 hip_check(ekgk::launch_class_sums(a, c, stream), "class_sums launch");
             }
         };

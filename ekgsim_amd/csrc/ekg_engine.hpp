@@ -74,9 +74,13 @@ struct Ctx {
     int kernel = EKG_KERNEL_AUTO;  // contraction path of the fused kernel
     bool graphs = false;           // replay repeated launch groups from a captured hipGraph
     int64_t graph_launches = 0, graph_captures = 0;
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;  // fused launches not yet timed
+    struct Timed {
+        hipEvent_t first, second;
+        bool counts;  // the first launch of its group
+    };
+    std::vector<Timed> pending;  // fused launches not yet timed
     std::vector<hipEvent_t> free_events;
-    int64_t fused_launches = 0;
+    int64_t fused_launches = 0;  // groups timed
     double fused_ms = 0.0;
     DevBuf nb_table;  // [4][26][4] int8 {d0, d1, d2, cube bit} of the four dipole neighbourhoods
     DevBuf crit_tg, crit_off, crit_stats, crit_out;  // criteria: targets, offsets, target statistics, output

@@ -66,8 +66,8 @@ int ekg_ctx_create(int device, ekg_ctx **out);
 void ekg_ctx_destroy(ekg_ctx *ctx);
 /* Kernel timing on the context stream: when enabled, every launch of the
  * fused AP+lead kernel is bracketed by HIP events; ekg_ctx_kernel_time
- * returns the number of launches and their summed duration since the last
- * reset. */
+ * returns the number of launch groups and the summed duration of their
+ * launches since the last reset. */
 int ekg_ctx_set_profiling(ekg_ctx *ctx, int enable);
 int ekg_ctx_kernel_time(ekg_ctx *ctx, const char *kernel, int64_t *launches, double *total_ms);
 int ekg_ctx_reset_profiling(ekg_ctx *ctx);
