@@ -1822,8 +1822,9 @@ __global__ __launch_bounds__(64 * CL_WAVES) void ecg_class_kernel(
         double v = s_acc[0][i][lane], c0 = 0.0;
 #pragma unroll
         for (int ww = 1; ww < HW; ++ww) v += s_acc[ww][i][lane];
+        const int np = H.n_classes < NP ? H.n_classes : NP;  // the other parts hold 0
 #pragma unroll 8
-        for (int p = 0; p < NP; ++p) c0 += s_k0[p][i];
+        for (int p = 0; p < np; ++p) c0 += s_k0[p][i];
         ecg[R.ecg_off + (int64_t)i * R.T + j] += v + c0;
     }
 }

@@ -1107,15 +1107,19 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
             const EcgLayout& hl = g.reqs[r].h->layout;
             int r1 = r;
             const int rg_first = (int)rgseg.size();
+            size_t at = rowtab.size(), leads = 0;
             for (; r1 < B && g.reqs[r1].h == g.reqs[r].h; ++r1)
-                if (hl.n_classes > 0)
-                    for (int i = 0; i < g.reqs[r1].L; ++i) {
-                        rowtab.push_back(r1 << 5 | i);
-                        rowpos.push_back((int)rd[r1].pos_off + 3 * i);
-                    }
-            while (rowtab.size() & 15) {
-                rowtab.push_back(rowtab.back() | (int)0x80000000u);
-                rowpos.push_back(rowpos.back());
+                if (hl.n_classes > 0) leads += g.reqs[r1].L;
+            rowtab.resize(at + ((leads + 15) & ~(size_t)15));
+            rowpos.resize(rowtab.size());
+            for (int q = r; q < r1 && leads > 0; ++q)
+                for (int i = 0; i < g.reqs[q].L; ++i, ++at) {
+                    rowtab[at] = q << 5 | i;
+                    rowpos[at] = (int)rd[q].pos_off + 3 * i;
+                }
+            for (; at < rowtab.size(); ++at) {
+                rowtab[at] = rowtab[at - 1] | (int)0x80000000u;
+                rowpos[at] = rowpos[at - 1];
             }
             const int64_t lines = std::max(1, hl.n_lines[g.nhood]);
             const int rg_end = (int)(rowtab.size() / 16);
@@ -1146,6 +1150,8 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
     // tables: uploaded only when they changed since the last group on this
     // workspace (a repeated group replays without host traffic)
     std::vector<char> tables;
+    tables.reserve(hdev.size() * sizeof hdev[0] + rd.size() * sizeof rd[0] + 7 * (B + 1) * 8 +
+                   segs.size() * sizeof(ekgk::ClassSeg) + (rgseg.size() + rowtab.size() + rowpos.size()) * 4);
     append(tables, hdev.data(), hdev.size());
     const size_t o_req = tables.size();
     append(tables, rd.data(), rd.size());
