@@ -1386,7 +1386,10 @@ __global__ void ecg_reduce_parts_kernel(const HeartDev* __restrict__ hearts, con
 // classes) for 16 leads; wave w takes boxes w, w + 4, ... (ordered by the host so
 // that the waves' work is equal) and adds their class sums into its own
 // LDS rows in order, then the waves' rows are added in wave order into
-// gsum[line of (region, class)][lead].  The cut into regions and the order
+// gsum[line of (region, class)][lead].  On hearts with many classes to a box the waves
+// divide the classes into 2 or 4 parts instead (each with its own LDS rows), and
+// the groups of waves of all parts the boxes: regions of 96 classes would hold one
+// or two boxes there (figures at class_cut).  The cut into regions and the order
 // depend on the heart only, so a request's bits do not depend on its batch.
 // Measured per 256 x 12 launch on the 128^3 heart: 0.83 ms (vector instructions
 // 0.52 and matrix products 0.15 of it), against 1.37 ms with the weights
@@ -1490,8 +1493,8 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     using gi32x4 = __attribute__((address_space(1))) const i32x4;
     using gint = __attribute__((address_space(1))) const int;
     using gf64 = __attribute__((address_space(1))) const double;
-    const i32x4 reg = ((ci32x4*)H.cregion)[2 * k];      // {first box, end box, first line, lines}
-    const i32x4 ext = ((ci32x4*)H.cregion)[2 * k + 1];  // {z0 | z1 << 16, y0 | y1 << 16, x0 | x1 << 16, 0}: cells + 1
+    const i32x4 reg = ((ci32x4*)H.cregion)[2 * k];      // {first box, end box, first line, lines | parts << 16}
+    const i32x4 ext = ((ci32x4*)H.cregion)[2 * k + 1];  // {z0 | z1 << 16, y0 | y1 << 16, x0 | x1 << 16: cells + 1, parts' first lines}
     gi32x4* const pkt = (gi32x4*)H.cbox + lane;
     gi32x4* const ini = (gi32x4*)H.cinit + lane;
     const char* const coef = (const char*)H.ccoef;
@@ -1654,10 +1657,13 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
         }
         __syncthreads();
         double* out = gsum + (sg.goff + (int64_t)rg * n_lines + reg.z) * 16;
-        for (int i = t; i < reg.w * 16; i += 64 * CB_WAVES) {
+        const int split = reg.w >> 16, l1 = ext.w & 511, l2 = (ext.w >> 9) & 511, l3 = ext.w >> 18;
+        for (int i = t; i < (reg.w & 0xffff) * 16; i += 64 * CB_WAVES) {
+            const int ln = i >> 4;
+            const int p = (ln >= l1) + (ln >= l2) + (ln >= l3);
+            const int slot = ln - (ln >= l3 ? l3 : ln >= l2 ? l2 : ln >= l1 ? l1 : 0);
             double v = 0.0;
-#pragma unroll
-            for (int q = 0; q < CB_WAVES; ++q) v += (&s_acc[q][0][0])[i];
+            for (int q = p; q < CB_WAVES; q += split) v += s_acc[q][slot][i & 15];
             out[i] = v;
         }
         __syncthreads();

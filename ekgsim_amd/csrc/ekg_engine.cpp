@@ -261,9 +261,7 @@ constexpr int64_t CLASS_CHUNK = 4096;
 // its share of class sums.
 constexpr int CLASS_WINDOW = 6;
 constexpr int64_t CLASS_PIECE = 1024;
-// Class boxes: 4 x 8 x 8 cells (z, y, x) in four sub-bricks of 4^3; a region
-// takes about 1/64 of a heart's boxes, at least 4 (one per wave of its block)
-// and at most 64.
+// Class boxes: 4 x 8 x 8 cells (z, y, x) in four sub-bricks of 4^3.
 constexpr int BOX_Z = 4, BOX_Y = 8, BOX_X = 8;
 constexpr int CB_SLOTS = ekgk::CB_SLOTS;
 constexpr int LONG_RANGES = 512;        // chunks from which the reduction sums in parts
@@ -585,11 +583,46 @@ void ensure_layout(Heart& h, bool mfma)
 //    (|D| <= 9 and, for any set of neighbours, |K| <= 93).  The kernel
 //    feeds each byte of a weight less 128, so a tile's accumulators start at 128
 //    times the sum of their coefficients.
-//  * Consecutive boxes form regions with at most CB_SLOTS classes, whose sums
-//    a block keeps in LDS; a box with more classes is listed again with the rest.
+//  * Consecutive boxes form regions, whose class sums a block keeps in LDS: at
+//    most CB_SLOTS classes, or on hearts with many classes to a box CB_SLOTS for each
+//    of 2 or 4 parts that the waves divide (class_cut); a box with more classes is
+//    listed again with the rest.  With parts, a box is listed once a part, with the
+//    part's classes.
 //    Each (region, class) has a line of sums, listed per class in order.
 // The cut depends on the heart only, so a request's ECG does not depend on
 // the batch it runs in.
+namespace {
+
+// Parts of a region's classes, and its boxes, from the mean number of classes of a box.
+// With few classes to a box a region holds boxes enough for its block's four
+// waves, each for all of the classes.  With many, one or two boxes fill the region's
+// slots, which leaves waves idle and a line of sums for almost every class of a
+// box; so the waves divide the classes, at the price of a box's weights once a
+// part, and the region holds as many times the classes.  Measured on
+// integer-delay hearts, us for 1 / 64 / 256 requests of 12 leads and 64 steps:
+//   classes a box   1 part               2 parts              4 parts
+//   112^3, 27       100 / 330 / 1,165     89 / 368 / 1,288    107 / 515 / 1,788
+//   144^3, 34       124 / 889 / -        104 / 758 / -        114 / 1,043 / -
+//   112^3, 37       100 / 482 / 1,786    100 / 422 / 1,474    121 / 561 / 2,001
+//   144^3, 43       145 / 1,245 / 4,816  123 / 795 / 2,909    136 / 1,094 / 3,957
+//   112^3, 62       120 / 1,151 / 4,426  119 / 691 / 2,432    152 / 723 / 2,589
+//   144^3, 73       201 / 3,710 / 14,434 161 / 1,568 / 5,981  182 / 1,436 / 5,230
+// Larger regions have fewer lines, smaller ones more blocks for a lone request:
+// 80^3 with 50 classes a box and two parts, 92 / 281 / 921 us with 8 boxes,
+// 92 / 277 / 898 with 12, 98 / 267 / 830 with 16.
+struct Cut {
+    int split, boxes;
+};
+
+Cut class_cut(int64_t pairs, int64_t boxes)
+{
+    const int split = pairs <= 33 * boxes ? 1 : pairs <= 70 * boxes ? 2 : 4;
+    if (split == 1) return {1, (int)std::min<int64_t>(64, std::max<int64_t>(4, (boxes / 64 + 3) / 4 * 4))};
+    return {split, (int)std::min<int64_t>(16, std::max<int64_t>(split == 2 ? 12 : 8, boxes / 192))};
+}
+
+}  // namespace
+
 void ensure_cells(Heart& h, int nhood)
 {
     EcgLayout& L = h.layout;
@@ -694,45 +727,97 @@ void ensure_cells(Heart& h, int nhood)
     std::vector<int8_t> coef;                 // 1024 per block
     std::vector<uint64_t> mask;               // 4 per listed box
     std::vector<std::pair<int, int>> lines;   // (class, line)
-    std::vector<int> slot_of(L.n_classes, -1), slot_cls;  // slots of the current region
-    const int target = (int)std::min<size_t>(64, std::max<size_t>(4, (order.size() / 64 + 3) / 4 * 4));
-    std::vector<int> cost;  // per listed box of the current region
+    // A region's classes are divided over `split` parts with CB_SLOTS slots each:
+    // wave w of a block adds the classes of part w % split, of every
+    // (CB_WAVES / split)-th box.
+    int64_t pairs = 0;  // (box, class)
+    for (size_t q = 0; q < sorted.size(); ++q)
+        pairs += q == 0 || sorted[q].box != sorted[q - 1].box || sorted[q].cls != sorted[q - 1].cls;
+    const Cut cut = class_cut(pairs, (int64_t)order.size());
+    const int split = cut.split, target = cut.boxes;
+    const int groups = ekgk::CB_WAVES / split;
+    std::vector<int> slot_of(L.n_classes, -1);     // part << 8 | slot in the current region
+    std::vector<std::vector<int>> slot_cls(split);  // the region's classes by part and slot
+    std::vector<int> cost;  // per item (box listing, one packet a part) of the current region
     auto close = [&]() {
         int4& r = regions.back();
         r.y = n_box;
-        // The block's wave w takes boxes w, w + 4, ...: order them so that
-        // the waves' work is about equal (largest first, each to the wave with
-        // least so far that still has a place).
-        const int n = r.y - r.x, nw = ekgk::CB_WAVES;
+        // Group g of the block's waves takes items g, g + groups, ...: order
+        // them so that the groups' work is about equal (largest first, each to
+        // the group with least so far that still has a place).
+        const int n = (r.y - r.x) / split;
         std::vector<int> by(n), at(n);
         std::iota(by.begin(), by.end(), 0);
         std::stable_sort(by.begin(), by.end(), [&](int x, int y) { return cost[x] > cost[y]; });
-        std::vector<int64_t> load(nw, 0);
-        std::vector<int> cnt(nw, 0);
+        std::vector<int64_t> load(groups, 0);
+        std::vector<int> cnt(groups, 0);
         for (int i : by) {
             int w = -1;
-            for (int q = 0; q < nw; ++q)
-                if (cnt[q] * nw + q < n && (w < 0 || load[q] < load[w])) w = q;
-            at[i] = cnt[w]++ * nw + w;
+            for (int q = 0; q < groups; ++q)
+                if (cnt[q] * groups + q < n && (w < 0 || load[q] < load[w])) w = q;
+            at[i] = cnt[w]++ * groups + w;
             load[w] += cost[i];
         }
         cost.clear();
         auto reorder = [&](auto& v, size_t per) {
             std::remove_reference_t<decltype(v)> tmp(v.begin() + (std::ptrdiff_t)(per * r.x), v.end());
+            per *= split;
             for (int i = 0; i < n; ++i)
-                std::copy_n(tmp.begin() + (std::ptrdiff_t)(per * i), per, v.begin() + (std::ptrdiff_t)(per * (r.x + at[i])));
+                std::copy_n(tmp.begin() + (std::ptrdiff_t)(per * i), per,
+                            v.begin() + (std::ptrdiff_t)(per / split * r.x + per * at[i]));
         };
         reorder(pkt, 64);
         reorder(init, 256);
         reorder(mask, 4);
-        r.w = (int)slot_cls.size();
-        for (size_t i = 0; i < slot_cls.size(); ++i) {
-            lines.push_back({slot_cls[i], r.z + (int)i});
-            slot_of[slot_cls[i]] = -1;
+        // the parts' lines one after the other; the first line of parts 1 to 3 (or past the region's)
+        int base = 0, first = 0;
+        for (int p = 0; p < ekgk::CB_WAVES; ++p) {
+            if (p > 0) first |= (p < split ? base : 511) << (9 * (p - 1));  // at most 3 CB_SLOTS: 9 bits
+            if (p >= split) continue;
+            for (size_t i = 0; i < slot_cls[p].size(); ++i) {
+                lines.push_back({slot_cls[p][i], r.z + base + (int)i});
+                slot_of[slot_cls[p][i]] = -1;
+            }
+            base += (int)slot_cls[p].size();
+            slot_cls[p].clear();
         }
-        slot_cls.clear();
+        r.w = base | split << 16;
+        ext.back().w = first;
     };
-    std::vector<int> cls;   // the box's classes
+    std::vector<int> cls;                         // the box's classes
+    std::vector<const Rec*> cls_rec;              // their records: [cls_rec[c], cls_rec[c + 1])
+    std::vector<int> cls_sub;                     // and the sub-bricks of their cells
+    std::vector<std::vector<size_t>> part(split);  // of an item: indexes into cls by part
+    std::vector<size_t> fresh;                    // the item's classes new to the region
+    // takes classes from c0 on into the item's parts, at most BOX_CLASSES a part; false when the
+    // region has no slot left for one
+    auto take = [&](size_t c0, size_t& c1) {
+        for (auto& q : part) q.clear();
+        fresh.clear();
+        for (c1 = c0; c1 < cls.size(); ++c1) {
+            int p = slot_of[cls[c1]] >> 8;
+            if (slot_of[cls[c1]] < 0) {
+                p = -1;
+                for (int q = 0; q < split; ++q)
+                    if (slot_cls[q].size() < (size_t)CB_SLOTS && (p < 0 || part[q].size() < part[p].size())) p = q;
+            }
+            if (p >= 0 && part[p].size() == BOX_CLASSES) break;
+            if (p < 0) {
+                for (size_t c : fresh) {
+                    slot_cls[slot_of[cls[c]] >> 8].pop_back();
+                    slot_of[cls[c]] = -1;
+                }
+                return false;
+            }
+            if (slot_of[cls[c1]] < 0) {
+                slot_of[cls[c1]] = p << 8 | (int)slot_cls[p].size();
+                slot_cls[p].push_back(cls[c1]);
+                fresh.push_back(c1);
+            }
+            part[p].push_back(c1);
+        }
+        return true;
+    };
     for (const auto& ob : order) {
         const Rec* r0 = sorted.data() + box_begin[ob.second];
         const Rec* r1 = sorted.data() + box_begin[ob.second + 1];
@@ -740,8 +825,15 @@ void ensure_cells(Heart& h, int nhood)
         int last_win[256];
         std::fill(last_win, last_win + 256, -1);
         cls.clear();
+        cls_rec.clear();
+        cls_sub.clear();
         for (const Rec* r = r0; r < r1; ++r) {
-            if (cls.empty() || cls.back() != r->cls) cls.push_back(r->cls);
+            if (cls.empty() || cls.back() != r->cls) {
+                cls.push_back(r->cls);
+                cls_rec.push_back(r);
+                cls_sub.push_back(0);
+            }
+            cls_sub.back() |= 1 << (r->cell >> 6);
             const int w = r->cls / CLASS_WINDOW;
             if (last_win[r->cell] != w) {
                 last_win[r->cell] = w;
@@ -749,73 +841,67 @@ void ensure_cells(Heart& h, int nhood)
                 ++n_entries;
             }
         }
-        for (size_t c0 = 0; c0 < cls.size(); c0 += BOX_CLASSES) {
-            const size_t c1 = std::min(cls.size(), c0 + BOX_CLASSES);
-            size_t fresh = 0;
-            for (size_t c = c0; c < c1; ++c) fresh += slot_of[cls[c]] < 0;
-            if (regions.empty() || slot_cls.size() + fresh > (size_t)CB_SLOTS ||
-                n_box - regions.back().x >= target) {
+        cls_rec.push_back(r1);
+        for (size_t c0 = 0, c1; c0 < cls.size(); c0 = c1) {
+            if (regions.empty() || n_box - regions.back().x >= target * split || !take(c0, c1)) {
                 if (!regions.empty()) close();
                 regions.push_back(int4{n_box, 0, (int)lines.size(), 0});
                 ext.push_back(int4{0xffff, 0xffff, 0xffff, 0});
+                take(c0, c1);
             }
-            for (size_t c = c0; c < c1; ++c)
-                if (slot_of[cls[c]] < 0) {
-                    slot_of[cls[c]] = (int)slot_cls.size();
-                    slot_cls.push_back(cls[c]);
-                }
-            const size_t blk0 = coef.size() / 1024;
-            const int n_tile = (int)((c1 - c0 + 3) / 4);
-            const size_t pk = 64 * (size_t)n_box;
-            pkt.resize(pk + 64, int4{0, 0, 0, 0});
-            init.resize(256 * (size_t)n_box + 256, 0);
-            const Rec* r = r0;
-            while (r < r1 && r->cls < cls[c0]) ++r;
-            int used = 0;
-            uint64_t bm[4] = {0, 0, 0, 0};
-            for (int t = 0; t < n_tile; ++t) {
-                const size_t q0 = c0 + 4 * t, q1 = std::min(c1, q0 + 4);
-                unsigned slots = 0;
-                for (size_t q = q0; q < q0 + 4; ++q)
-                    slots |= (unsigned)(q < q1 ? slot_of[cls[q]] : CB_SLOTS) << (8 * (q - q0));
-                const Rec* rt = r;
-                int subs = 0;
-                for (; r < r1 && r->cls <= cls[q1 - 1]; ++r) subs |= 1 << (r->cell >> 6);
-                if (coef.size() / 1024 > 0x7ffffff0u) fail(EKG_EINVAL, "too many class cells");
-                const size_t base = coef.size(), ib = 256 * (size_t)n_box + 16 * t;
-                pkt[pk + t] = int4{subs, (int)slots, (int)(base / 1024), 0};
-                coef.resize(base + 1024 * (size_t)__builtin_popcount((unsigned)subs), 0);
-                size_t q = q0;
-                for (; rt < r; ++rt) {
-                    while (cls[q] != rt->cls) ++q;
-                    const int sub = rt->cell >> 6, z = (rt->cell >> 4) & 3, y = (rt->cell >> 2) & 3, x = rt->cell & 3;
-                    const int dz = z, dy = y + 4 * (sub >> 1), dx = x + 4 * (sub & 1);
-                    const int K = -(rt->d[0] * dz + rt->d[1] * dy + rt->d[2] * dx);
-                    if (K < -127 || K > 127) fail(EKG_EINVAL, "dipole moment out of range");
-                    const int row = 4 * (int)(q - q0);
-                    const int co[4] = {rt->d[0], rt->d[1], rt->d[2], K};
-                    const size_t blk = base + 1024 * (size_t)__builtin_popcount((unsigned)(subs & ((1 << sub) - 1)));
-                    bm[sub] |= (uint64_t)1 << (rt->cell & 63);
-                    used |= 1 << (4 * sub + y);
-                    for (int i = 0; i < 4; ++i) {
-                        coef[blk + 16 * (16 * z + row + i) + 4 * y + x] = (int8_t)co[i];
-                        init[ib + row + i] += 128 * co[i];
-                    }
-                }
-            }
+            int item_cost = 0;
             const int o[3] = {bz * BOX_Z + 1, by * BOX_Y + 1, bx * BOX_X + 1};
-            pkt[pk + 16] = int4{n_tile, used, 0, 0};
-            pkt[pk + 17] = int4{o[0], o[1], o[2], 0};
-            // cycles of a box, roughly: 34 a weight of 64 lanes, 64 a block's
-            // four products, 180 a tile's flush
-            cost.push_back(500 + 136 * __builtin_popcount((unsigned)used) +
-                           64 * (int)(coef.size() / 1024 - blk0) + 180 * n_tile);
-            ++n_box;
+            for (const std::vector<size_t>& pc : part) {
+                const size_t blk0 = coef.size() / 1024;
+                const int n_tile = std::max(1, (int)((pc.size() + 3) / 4));  // none: an empty tile
+                const size_t pk = 64 * (size_t)n_box;
+                pkt.resize(pk + 64, int4{0, 0, 0, 0});
+                init.resize(256 * (size_t)n_box + 256, 0);
+                int used = 0;
+                uint64_t bm[4] = {0, 0, 0, 0};
+                for (int t = 0; t < n_tile; ++t) {
+                    const size_t q0 = 4 * t, q1 = std::min(pc.size(), q0 + 4);
+                    unsigned slots = 0;
+                    int subs = 0;
+                    for (size_t q = q0; q < q0 + 4; ++q) {
+                        slots |= (unsigned)(q < q1 ? slot_of[cls[pc[q]]] & 255 : CB_SLOTS) << (8 * (q - q0));
+                        if (q < q1) subs |= cls_sub[pc[q]];
+                    }
+                    if (coef.size() / 1024 > 0x7ffffff0u) fail(EKG_EINVAL, "too many class cells");
+                    const size_t base = coef.size(), ib = 256 * (size_t)n_box + 16 * t;
+                    pkt[pk + t] = int4{subs, (int)slots, (int)(base / 1024), 0};
+                    coef.resize(base + 1024 * (size_t)__builtin_popcount((unsigned)subs), 0);
+                    for (size_t q = q0; q < q1; ++q)
+                        for (const Rec* r = cls_rec[pc[q]]; r < cls_rec[pc[q] + 1]; ++r) {
+                            const int sub = r->cell >> 6, z = (r->cell >> 4) & 3, y = (r->cell >> 2) & 3, x = r->cell & 3;
+                            const int dz = z, dy = y + 4 * (sub >> 1), dx = x + 4 * (sub & 1);
+                            const int K = -(r->d[0] * dz + r->d[1] * dy + r->d[2] * dx);
+                            if (K < -127 || K > 127) fail(EKG_EINVAL, "dipole moment out of range");
+                            const int row = 4 * (int)(q - q0);
+                            const int co[4] = {r->d[0], r->d[1], r->d[2], K};
+                            const size_t blk = base + 1024 * (size_t)__builtin_popcount((unsigned)(subs & ((1 << sub) - 1)));
+                            bm[sub] |= (uint64_t)1 << (r->cell & 63);
+                            used |= 1 << (4 * sub + y);
+                            for (int i = 0; i < 4; ++i) {
+                                coef[blk + 16 * (16 * z + row + i) + 4 * y + x] = (int8_t)co[i];
+                                init[ib + row + i] += 128 * co[i];
+                            }
+                        }
+                }
+                pkt[pk + 16] = int4{n_tile, used, 0, 0};
+                pkt[pk + 17] = int4{o[0], o[1], o[2], 0};
+                // cycles of a box, roughly: 34 a weight of 64 lanes, 64 a block's
+                // four products, 180 a tile's flush
+                item_cost = std::max(item_cost, 500 + 136 * __builtin_popcount((unsigned)used) +
+                                                    64 * (int)(coef.size() / 1024 - blk0) + 180 * n_tile);
+                ++n_box;
+                mask.insert(mask.end(), bm, bm + 4);
+            }
+            cost.push_back(item_cost);
             const int len[3] = {BOX_Z, BOX_Y, BOX_X};
             int* e = &ext.back().x;
             for (int i = 0; i < 3; ++i)
                 e[i] = std::min(e[i] & 0xffff, o[i]) | std::max(e[i] >> 16, o[i] + len[i] - 1) << 16;
-            mask.insert(mask.end(), bm, bm + 4);
         }
     }
     if (!regions.empty()) close();

@@ -76,11 +76,12 @@ struct HeartDev {
     const int4* classes;         // [n_classes] {layer, first class chunk, end class chunk, 0}
     const double* class_a;       // [n_classes] activation time of the class
     // class boxes for the group's neighbourhood (ensure_cells): regions
-    // {first box, end box, first line, lines} and {first | last << 16 cell + 1
-    // per axis}; per box 64 records (its tiles of 4 classes {sub-bricks, 4 slot bytes,
-    // first block, 0}, from 16 on {tiles, rows of 16 cells in use, 0, 0} and {first
-    // cell + 1}) and the 16 tiles' 16 accumulator starts; coefficient blocks of 64
-    // lanes x 16 bytes; per box and sub-brick the cells that carry dipoles; the lines
+    // {first box, end box, first line, lines | parts << 16} and {first | last << 16
+    // cell + 1 per axis, first lines of parts 1 to 3, 9 bits each}; per box 64
+    // records (its tiles of 4 classes {sub-bricks, 4 slot bytes, first block, 0},
+    // from 16 on {tiles, rows of 16 cells in use, 0, 0} and {first cell + 1}) and
+    // the 16 tiles' 16 accumulator starts; coefficient blocks of 64 lanes x 16
+    // bytes; per box and sub-brick the cells that carry dipoles; the lines
     // (region, slot) of class k are cs_line[cs_off[k] .. cs_off[k + 1])
     const int4* cregion;
     const int4* cbox;
