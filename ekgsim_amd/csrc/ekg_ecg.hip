@@ -1456,7 +1456,7 @@ __device__ __forceinline__ ScaleRange scale_range(float qz, float qy, float qx, 
 
 __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     const HeartDev* __restrict__ hearts, const ClassSeg* __restrict__ segs, int n_segs, const int* __restrict__ rowpos,
-    const double* __restrict__ lead_pos, double* __restrict__ gsum)
+    const double* __restrict__ lead_pos, double* __restrict__ gsum, int line0, int line1, int reg0, int n_reg)
 {
     __shared__ double s_acc[CB_WAVES][CB_SLOTS + 1][16];  // last row: classes past a tile's end
     __shared__ i32x4 s_init[CB_WAVES][64];
@@ -1476,7 +1476,8 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     // on XCD x with all its rows of 16 leads back to back, so that each region's
     // coefficients are fetched into one L2.  A block takes sg.per rows of a
     // region in turn (the chain of loads that starts a block, paid once).
-    const int local = (int)(blk - sg.block0), n8 = sg.n_regions >> 3, ns = (sg.n_rg + sg.per - 1) / sg.per;
+    const int nr = n_reg > 0 ? n_reg : sg.n_regions;
+    const int local = (int)(blk - sg.block0), n8 = nr >> 3, ns = (sg.n_rg + sg.per - 1) / sg.per;
     int k, rg;
     if (local < 8 * n8 * ns) {
         const int q = local >> 3;
@@ -1488,6 +1489,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
         rg = q % ns * sg.per;
     }
     const int rg_end = rg + sg.per < sg.n_rg ? rg + sg.per : sg.n_rg;
+    k += reg0;
     const HeartDev& H = hearts[sg.heart];
     using ci32x4 = __attribute__((address_space(4))) const i32x4;
     using gi32x4 = __attribute__((address_space(1))) const i32x4;
@@ -1498,7 +1500,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     gi32x4* const pkt = (gi32x4*)H.cbox + lane;
     gi32x4* const ini = (gi32x4*)H.cinit + lane;
     const char* const coef = (const char*)H.ccoef;
-    const int n_lines = H.n_lines;
+    const int n_lines = (line1 < H.n_lines ? line1 : H.n_lines) - line0;
     const int zq = lane >> 4;
     // electrode position offset of the lane's lead
     int po = ((gint*)rowpos)[16 * (sg.rg0 + rg) + (lane & 15)];
@@ -1656,15 +1658,16 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
             }
         }
         __syncthreads();
-        double* out = gsum + (sg.goff + (int64_t)rg * n_lines + reg.z) * 16;
+        double* const out = gsum + (sg.goff + (int64_t)rg * n_lines) * 16 + (t & 15);
         const int split = reg.w >> 16, l1 = ext.w & 511, l2 = (ext.w >> 9) & 511, l3 = ext.w >> 18;
         for (int i = t; i < (reg.w & 0xffff) * 16; i += 64 * CB_WAVES) {
-            const int ln = i >> 4;
+            const int ln = i >> 4, at = reg.z + ln - line0;
+            if ((unsigned)at >= (unsigned)n_lines) continue;  // a region that reaches past the launch's lines
             const int p = (ln >= l1) + (ln >= l2) + (ln >= l3);
             const int slot = ln - (ln >= l3 ? l3 : ln >= l2 ? l2 : ln >= l1 ? l1 : 0);
             double v = 0.0;
             for (int q = p; q < CB_WAVES; q += split) v += s_acc[q][slot][i & 15];
-            out[i] = v;
+            out[(int64_t)16 * at] = v;
         }
         __syncthreads();
     }
@@ -1674,12 +1677,15 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
 // lead) of a launch's 16-lead rows: k0 sum G, P' sum G, Q' sum G, with the
 // sum over the class's regions in order, k0 the class's layer's resting value
 // and P' = k2(1-k3) e^{(k4+k5)(a - t0)}, Q' = k2 k3 e^{k5 (a - t0)}.  The
-// thread of a request's last lead also clears the unused lead slots.
+// thread of a request's last lead also clears the unused lead slots.  A launch
+// over the lines [line0, line1) of a row goes on from the sum that the launch before
+// it left in csums; the factors come with the last (the same sum in the same
+// order, however the lines are cut).
 template <int LP>
 __global__ __launch_bounds__(256) void class_sums_kernel(
     const HeartDev* __restrict__ hearts, const ReqDev* __restrict__ reqs, const ClassSeg* __restrict__ segs,
     const int* __restrict__ rgseg, const int* __restrict__ rowtab, int rg0, const double* __restrict__ layer_k,
-    const double* __restrict__ gsum, double* __restrict__ csums)
+    const double* __restrict__ gsum, double* __restrict__ csums, int line0, int line1)
 {
     const int rg = rg0 + blockIdx.y, t = threadIdx.x;
     const ClassSeg sg = segs[rgseg[rg]];
@@ -1687,16 +1693,26 @@ __global__ __launch_bounds__(256) void class_sums_kernel(
     const int k = blockIdx.x * 16 + (t >> 4);
     const int row = rowtab[16 * rg + (t & 15)];
     if (k >= H.n_classes || row < 0) return;
-    const double* g = gsum + (sg.goff + (int64_t)(rg - sg.rg0) * H.n_lines) * 16 + (t & 15);
-    double s = 0.0;
-    const int q1 = H.cs_off[k + 1];
-#pragma unroll 8
-    for (int q = H.cs_off[k]; q < q1; ++q) s += g[(int64_t)16 * H.cs_line[q]];
     const ReqDev& R = reqs[row >> 5];
     const int i = row & 31, l = H.classes[k].x;
+    double* o = csums + (R.cls_off + k) * 3 * LP;
+    const bool whole = line0 == 0 && line1 >= H.n_lines;
+    const int stride = whole ? H.n_lines : (line1 < H.n_lines ? line1 : H.n_lines) - line0;
+    const double* g = gsum + (sg.goff + (int64_t)(rg - sg.rg0) * stride - line0) * 16 + (t & 15);
+    double s = line0 > 0 ? o[i] : 0.0;
+    int q0 = H.cs_off[k], q1 = H.cs_off[k + 1];
+    if (!whole) {  // a class's lines ascend
+        while (q0 < q1 && H.cs_line[q0] < line0) ++q0;
+        while (q0 < q1 && H.cs_line[q1 - 1] >= line1) --q1;
+    }
+#pragma unroll 8
+    for (int q = q0; q < q1; ++q) s += g[(int64_t)16 * H.cs_line[q]];
+    if (line1 < H.n_lines) {
+        o[i] = s;
+        return;
+    }
     const double* kk = layer_k + R.k_off + 9 * (l - 1);
     const double da = H.class_a[k] - H.layer_t0[l];
-    double* o = csums + (R.cls_off + k) * 3 * LP;
     o[i] = s * kk[0];
     o[LP + i] = kk[2] * (1.0 - kk[3]) * exp((kk[4] + kk[5]) * da) * s;
     o[2 * LP + i] = kk[2] * kk[3] * exp(kk[5] * da) * s;
@@ -2002,7 +2018,7 @@ hipError_t launch_class_boxes(const GroupArgs& a, const ClassLaunch& c, hipStrea
     if (c.blocks < 0 || c.blocks > 0x7fffffffLL || c.n_segs < 1) return hipErrorInvalidValue;
     if (c.blocks == 0) return hipSuccess;  // hearts without class cells: their sums are zero
     hipLaunchKernelGGL(ecg_class_box_kernel, dim3((unsigned)c.blocks), dim3(64 * CB_WAVES), 0, s, a.hearts,
-                       a.segs + c.seg0, c.n_segs, a.rowpos, a.lead_pos, a.gsum);
+                       a.segs + c.seg0, c.n_segs, a.rowpos, a.lead_pos, a.gsum, c.l0, c.l1, c.reg0, c.n_reg);
     return hipGetLastError();
 }
 
@@ -2014,7 +2030,7 @@ hipError_t launch_class_sums(const GroupArgs& a, const ClassLaunch& c, hipStream
     case LPV:                                                                                                \
         hipLaunchKernelGGL(class_sums_kernel<LPV>, dim3((unsigned)((a.cs_max + 15) / 16), (unsigned)c.n_rg), \
                            dim3(256), 0, s, a.hearts, a.reqs, a.segs, a.rgseg, a.rowtab, c.rg0, a.layer_k,   \
-                           a.gsum, a.csums);                                                                 \
+                           a.gsum, a.csums, c.l0, c.l1);                                                     \
         break;
         EKG_CSUMS(4)
         EKG_CSUMS(8)

@@ -940,6 +940,9 @@ void ensure_cells(Heart& h, int nhood)
     L.n_centries[nhood] = n_entries;
     L.n_cpieces[nhood] = (int)n_pieces;
     L.n_lines[nhood] = (int)lines.size();
+    L.h_region_line[nhood].clear();
+    for (const int4& r : regions) L.h_region_line[nhood].push_back(r.z);
+    L.h_region_line[nhood].push_back((int)lines.size());
     L.n_regions[nhood] = (int)regions.size();
     L.cells_built[nhood] = true;
 }
@@ -975,13 +978,19 @@ void append(std::vector<char>& buf, const T* p, size_t n)
     buf.insert(buf.end(), c, c + n * sizeof(T));
 }
 
-// Lines of a group's class sums, and the most of one row: the leads of each run
-// of consecutive requests of one heart fill rows of 16, a row has a line per
-// (region, class) of the heart.  Before the cells are built, each class counts in an
-// eighth of the regions; a heart that is one class as a whole (no lines: its
-// cells cancel) counts one.
+// Lines of a group's class sums: the leads of each run of consecutive requests
+// of one heart fill rows of 16, a row has a line per (region, class) of the
+// heart.  Before the cells are built, a class counts eight lines (2 to 45 on hearts
+// measured: a guess, which a launch is held to by class_bytes); a heart that is one class as a
+// whole (no lines: its cells cancel) counts one.
 struct ClassLines {
-    int64_t all = 0, row = 0;
+    int64_t all = 0, rows = 0, runs = 0;
+    // most bytes of the rows' tables: row and position of 16 leads, segment
+    // of each row, and a segment per run and launch
+    int64_t table_bytes(int64_t cap) const
+    {
+        return rows * (16 * 8 + 4) + std::min(rows, runs + 1 + 2 * all / cap) * (int64_t)sizeof(ekgk::ClassSeg);
+    }
 };
 
 ClassLines class_lines(const GroupPlan& g)
@@ -996,14 +1005,15 @@ ClassLines class_lines(const GroupPlan& g)
         if (!(g.mfma && L.valid && L.n_classes > 0)) continue;
         const int64_t lines = L.cells_built[g.nhood] ? std::max(1, L.n_lines[g.nhood]) : (int64_t)8 * L.n_classes;
         c.all += (leads + 15) / 16 * lines;
-        c.row = std::max(c.row, lines);
+        c.rows += (leads + 15) / 16;
+        ++c.runs;
     }
     return c;
 }
 
 }  // namespace
 
-size_t group_device_bytes(const GroupPlan& g)
+size_t group_device_bytes(GroupPlan& g)
 {
     size_t s = 0;
     const int LP = g.LP;
@@ -1024,11 +1034,13 @@ size_t group_device_bytes(const GroupPlan& g)
              (8 + 2 * LP * 8);
         s += (size_t)nmix * LP * r.Tp * 8;
         s += (size_t)r.L * r.T * 8;
-        // record, heart, seven start tables, class rows
-        s += sizeof(ekgk::ReqDev) + sizeof(ekgk::HeartDev) + 7 * 8 + sizeof(ekgk::ClassSeg) + r.L * 12;
+        // record, heart, seven start tables
+        s += sizeof(ekgk::ReqDev) + sizeof(ekgk::HeartDev) + 7 * 8;
     }
     const ClassLines c = class_lines(g);
-    return s + (size_t)std::max(c.row * LINE_BYTES, std::min(c.all * LINE_BYTES, GSUM_BYTES));
+    g.class_bytes = std::min(c.all * LINE_BYTES, GSUM_BYTES);
+    if (c.all == 0) return s;
+    return s + (size_t)(c.table_bytes(1) + g.class_bytes);
 }
 
 void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, const double* d_k,
@@ -1186,7 +1198,9 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         const ClassLines cl = class_lines(g);
         int64_t fixed = 0;
         for (const ReqSpec& r : g.reqs) fixed += fixed_class_bytes(r, LP);
-        const int64_t cap = std::max(cl.row, ws.arena ? fixed / LINE_BYTES : std::min(cl.all, GSUM_BYTES / LINE_BYTES));
+        int64_t cap = ws.arena ? fixed / LINE_BYTES : std::min(cl.all, GSUM_BYTES / LINE_BYTES);
+        if (g.class_bytes >= 0) cap = std::min(cap, g.class_bytes / LINE_BYTES);
+        cap = std::max<int64_t>(1, cap);
         ws.need(ws.gsum, (size_t)(cap * LINE_BYTES));
         int64_t block0 = 0, used = cap;  // lines taken in the current launch
         for (int r = 0; r < B;) {
@@ -1210,8 +1224,25 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
             const int64_t lines = std::max(1, hl.n_lines[g.nhood]);
             const int rg_end = (int)(rowtab.size() / 16);
             for (int rg = rg_first; rg < rg_end;) {
+                if (lines > cap) {  // not even one row fits: its lines in turn, cut at regions where that leaves half
+                    const std::vector<int>& rl = hl.h_region_line[g.nhood];
+                    for (int64_t l0 = 0, l1; l0 < lines; l0 = l1) {
+                        l1 = std::min(lines, l0 + cap);
+                        const int cut = *(std::upper_bound(rl.begin(), rl.end(), (int)l1) - 1);
+                        if (cut - l0 >= cap / 2 && cut > l0) l1 = cut;
+                        const int reg0 = (int)(std::upper_bound(rl.begin(), rl.end(), (int)l0) - rl.begin()) - 1;
+                        const int reg1 = (int)(std::lower_bound(rl.begin(), rl.end(), (int)l1) - rl.begin());
+                        launches.push_back({(int)segs.size(), 1, rg, 1, (int)l0, (int)l1, reg0, reg1 - reg0, reg1 - reg0});
+                    }
+                    segs.push_back(ekgk::ClassSeg{rg, 1, hl.n_regions[g.nhood], rd[r].heart, 1, 0, block0, 0});
+                    rgseg.push_back((int)segs.size() - 1);
+                    block0 += hl.n_regions[g.nhood];
+                    used = cap;
+                    ++rg;
+                    continue;
+                }
                 if (used + lines > cap || launches.back().n_rg >= 65535) {
-                    launches.push_back(ekgk::ClassLaunch{(int)segs.size(), 0, rg, 0, 0});
+                    launches.push_back({(int)segs.size(), 0, rg, 0});
                     used = 0;
                 }
                 ekgk::ClassLaunch& la = launches.back();

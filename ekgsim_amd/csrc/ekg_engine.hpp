@@ -117,6 +117,7 @@ struct EcgLayout {
     bool cells_built[4] = {false, false, false, false};
     int64_t n_ccells[4] = {0, 0, 0, 0}, n_centries[4] = {0, 0, 0, 0};
     int n_cpieces[4] = {0, 0, 0, 0}, n_lines[4] = {0, 0, 0, 0}, n_regions[4] = {0, 0, 0, 0};
+    std::vector<int> h_region_line[4];  // first line of each region, then their end
     DevBuf cregion[4], cbox[4], cinit[4], ccoef[4], cmask[4], cs_off[4], cs_line[4];
     std::vector<int> h_layer_chunk;
     std::vector<double> h_layer_t0;
@@ -160,6 +161,7 @@ struct GroupPlan {
     std::vector<ReqSpec> reqs;
     int LP = 4, nhood = 0, waves = 2, lf_phase = 2;
     bool mfma = true;
+    int64_t class_bytes = -1;  // most bytes of class sums a launch may take (-1: as the group needs)
 };
 
 int nhood_offsets(int type, int8_t dif[26][3]);
@@ -178,7 +180,8 @@ bool layout_ready(const Heart& h, bool mfma, int nhood);
 void ensure_cells(Heart& h, int nhood);
 // Whether the heart's simulations take the matrix-core path (as plan_group decides).
 bool heart_mfma(const Ctx& ctx, const Heart& h);
-size_t group_device_bytes(const GroupPlan& g);
+// Device bytes of the group; sets class_bytes to the share of its class sums in them.
+size_t group_device_bytes(GroupPlan& g);
 // Enqueue a whole group on `stream`.  With d_k/d_pos null the host values of
 // the specs are packed and uploaded; otherwise request r reads
 // d_k[r*nl*9 ...] and d_pos[r*L*3 ...] (uniform device batches).  ECGs go to

@@ -122,10 +122,12 @@ struct ClassSeg {
     int64_t block0, goff;
 };
 // One launch of the class-box and class-sum kernels: segments whose sums fit
-// gsum together.
+// gsum together, or, where not even a row's lines do, the lines [l0, l1) of one
+// row, from its regions [reg0, reg0 + n_reg).
 struct ClassLaunch {
     int seg0, n_segs, rg0, n_rg;
-    int64_t blocks;
+    int l0 = 0, l1 = 0x7fffffff, reg0 = 0, n_reg = 0;  // n_reg 0: all lines and regions
+    int64_t blocks = 0;
 };
 
 // A launch group: requests of any hearts, lead counts and time grids that
