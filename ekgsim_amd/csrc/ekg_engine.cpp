@@ -511,13 +511,9 @@ void ensure_layout(Heart& h, bool mfma)
         hip_check(hipMemcpy(L.chunks.p, L.h_chunks.data(), L.h_chunks.size() * sizeof(int4),
                             hipMemcpyHostToDevice),
                   "upload chunks");
-    L.cchunks.reserve(std::max<size_t>(1, L.h_cchunks.size()) * sizeof(int4));
     L.classes.reserve(std::max<size_t>(1, L.h_classes.size()) * sizeof(int4));
     L.class_a.reserve(std::max<size_t>(1, L.h_class_a.size()) * sizeof(double));
     if (!L.h_cchunks.empty()) {
-        hip_check(hipMemcpy(L.cchunks.p, L.h_cchunks.data(), L.h_cchunks.size() * sizeof(int4),
-                            hipMemcpyHostToDevice),
-                  "upload class chunks");
         hip_check(hipMemcpy(L.classes.p, L.h_classes.data(), L.h_classes.size() * sizeof(int4),
                             hipMemcpyHostToDevice),
                   "upload classes");
@@ -547,7 +543,6 @@ void ensure_layout(Heart& h, bool mfma)
     d.chunks = L.chunks.as<int4>();
     d.layer_chunk = L.layer_chunk.as<int>();
     d.layer_t0 = L.layer_t0.as<double>();
-    d.cchunks = L.cchunks.as<int4>();
     d.classes = L.classes.as<int4>();
     d.class_a = L.class_a.as<double>();
     d.n0 = h.n0;
@@ -557,7 +552,6 @@ void ensure_layout(Heart& h, bool mfma)
     d.n_chunks = L.n_chunks;
     d.n_bricks = L.n_bricks;
     d.max_layer = h.max_layer;
-    d.n_cchunks = L.n_cchunks;
     d.n_classes = L.n_classes;
     L.valid = true;
 }
@@ -1013,7 +1007,7 @@ ClassLines class_lines(const GroupPlan& g)
 
 }  // namespace
 
-size_t group_device_bytes(GroupPlan& g)
+size_t group_device_bytes(GroupPlan& g, size_t budget)
 {
     size_t s = 0;
     const int LP = g.LP;
@@ -1040,7 +1034,11 @@ size_t group_device_bytes(GroupPlan& g)
     const ClassLines c = class_lines(g);
     g.class_bytes = std::min(c.all * LINE_BYTES, GSUM_BYTES);
     if (c.all == 0) return s;
-    return s + (size_t)(c.table_bytes(1) + g.class_bytes);
+    // a row of class sums is cut into as many launches as its share asks for, down to a line each
+    const int64_t tables = c.table_bytes(1);
+    if (s + (size_t)(tables + g.class_bytes) > budget)
+        g.class_bytes = std::max<int64_t>(LINE_BYTES, (int64_t)budget - (int64_t)s - tables) / LINE_BYTES * LINE_BYTES;
+    return s + (size_t)(tables + g.class_bytes);
 }
 
 void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, const double* d_k,

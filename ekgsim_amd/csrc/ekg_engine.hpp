@@ -122,7 +122,7 @@ struct EcgLayout {
     std::vector<int> h_layer_chunk;
     std::vector<double> h_layer_t0;
     DevBuf vox_chunk, vox_a64, vox_a, vox_geo, chunks, bricks, brick_off, brick_vox, halo_off, halo_cells,
-        layer_chunk, layer_t0, cchunks, classes, class_a;
+        layer_chunk, layer_t0, classes, class_a;
     ekgk::HeartDev dev{};          // device pointers and sizes for the kernels
 };
 struct Heart {
@@ -180,8 +180,9 @@ bool layout_ready(const Heart& h, bool mfma, int nhood);
 void ensure_cells(Heart& h, int nhood);
 // Whether the heart's simulations take the matrix-core path (as plan_group decides).
 bool heart_mfma(const Ctx& ctx, const Heart& h);
-// Device bytes of the group; sets class_bytes to the share of its class sums in them.
-size_t group_device_bytes(GroupPlan& g);
+// Device bytes of the group, at most `budget` if its class sums can be cut to that
+// (they then take more launches): sets class_bytes to their share.
+size_t group_device_bytes(GroupPlan& g, size_t budget = SIZE_MAX);
 // Enqueue a whole group on `stream`.  With d_k/d_pos null the host values of
 // the specs are packed and uploaded; otherwise request r reads
 // d_k[r*nl*9 ...] and d_pos[r*L*3 ...] (uniform device batches).  ECGs go to

@@ -69,10 +69,7 @@ struct HeartDev {
     const int* layer_chunk;      // [max_layer + 2]: chunks of layer l are [layer_chunk[l], layer_chunk[l+1])
     const double* layer_t0;      // [max_layer + 1]: reference time of layer l
     // Activation classes: runs of one layer and one activation time, whose
-    // voxels all have the same AP.  Their voxels are cut into class chunks
-    // (index n_chunks + k of the per-chunk sums); the chunks above hold the
-    // other voxels.
-    const int4* cchunks;         // [n_cchunks] {layer, v_begin, v_end, t_ref as float bits}
+    // voxels all have the same AP; the chunks above hold the other voxels.
     const int4* classes;         // [n_classes] {layer, first class chunk, end class chunk, 0}
     const double* class_a;       // [n_classes] activation time of the class
     // class boxes for the group's neighbourhood (ensure_cells): regions
@@ -93,7 +90,7 @@ struct HeartDev {
     int n_lines, n_regions;
     int n0, n1, n2;
     int V, n_chunks, n_bricks, max_layer;
-    int n_cchunks, n_classes;
+    int n_classes;
 };
 
 // One request of a launch group.  Offsets index the group's packed arrays.

@@ -294,6 +294,10 @@ void Server::run()
                     launched = true;
                 }
             }
+            // a lone request that does not fit with its class sums in one
+            // launch takes what is left for them
+            if (ok && inflight == 0 && bytes_in_use + bytes > opts.hbm_budget_bytes && bytes_in_use < opts.hbm_budget_bytes)
+                bytes = group_device_bytes(plan, opts.hbm_budget_bytes - bytes_in_use);
             if (ok && bytes_in_use + bytes > opts.hbm_budget_bytes) {
                 if (inflight == 0) {
                     std::vector<Request*> one{head};

@@ -1,5 +1,6 @@
 """Device memory of server groups against what they are accounted as: a heart whose class
-layout an excitation dropped (it is sized before the layout exists again)."""
+layout an excitation dropped (it is sized before the layout exists again), and budgets that held a
+request before class sums were kept per region."""
 import numpy as np
 import pytest
 
@@ -38,3 +39,53 @@ def test_request_of_a_reexcited_heart_takes_what_is_accounted():
     # the same buffers but for the class sums: what is accounted less is taken less (the
     # allocator rounds to 2 MiB)
     assert used[2] <= used[1] - (peak[1] - peak[2]) + 4 * MIB
+
+
+# Bytes of one request of 200 steps on these hearts as they were accounted when a class took
+# three sums per lead slot and piece of a window of classes: grid, leads, budget.
+BUDGETS = [(24, 2, 88848), (24, 12, 240128), (24, 16, 314144), (48, 2, 95136), (48, 12, 258512), (48, 16, 338576),
+           (96, 2, 105320), (96, 12, 287064), (96, 16, 376312)]
+
+
+@pytest.mark.parametrize("n,leads,budget", BUDGETS)
+def test_budget_that_held_a_request_still_does(n, leads, budget):
+    ctx = E.Context(0)
+    h = S.make_heart(n, seed=1)
+    g = E.Heart(ctx, h.layer, h.seed)
+    g.excite_delay(h.delay)
+    k = S.layer_k_from_params(S.random_params(3, 1, 11), 3)
+    pos = S.lead_positions(n, leads)
+    ref = g.simulate(k, pos, "3D4", 0.0, 200.0, 1.0)
+    srv = E.Server(ctx, hbm_budget_bytes=budget)
+    hid = srv.add_heart(g)
+    tickets = [srv.submit(hid, k, pos, "3D4", 0.0, 200.0, 1.0) for _ in range(3)]
+    for t in tickets:
+        assert np.array_equal(srv.wait(t)[0], ref)
+    print(f"{n}^3, {leads} leads: budget {budget}, peak {srv.stats()['peak_bytes']}")
+    assert srv.stats()["peak_bytes"] <= budget
+    srv.close()
+    # a budget too small for the request without its class sums is refused, as before
+    srv = E.Server(ctx, hbm_budget_bytes=budget // 2)
+    hid = srv.add_heart(g)
+    with pytest.raises(E.EkgError) as e:
+        srv.wait(srv.submit(hid, k, pos, "3D4", 0.0, 200.0, 1.0))
+    assert e.value.code == 2  # EKG_ENOMEM
+    srv.close()
+    g.close()
+    ctx.close()
+
+
+def test_budget_that_held_a_request_with_one_class_still_does():
+    ctx = E.Context(0)
+    n, budget = 64, 9086976  # one small class among 363 chunks
+    h = S.make_heart(n, seed=1)
+    g = E.Heart(ctx, h.layer, h.seed)
+    g.excite_transfer(S.layered_transfer(3, 5, diag=1.03, off=1.57))
+    k = S.layer_k_from_params(S.random_params(3, 1, 11), 3)
+    srv = E.Server(ctx, hbm_budget_bytes=budget)
+    hid = srv.add_heart(g)
+    srv.wait(srv.submit(hid, k, S.lead_positions(n, 12), "3D4", 0.0, 200.0, 1.0))
+    assert srv.stats()["peak_bytes"] <= budget
+    srv.close()
+    g.close()
+    ctx.close()
