@@ -69,12 +69,16 @@ void Workspace::need(DevBuf& b, size_t n)
         return;
     }
     const size_t at = (arena_used + 255) & ~(size_t)255;
-    if (at > arena_bytes || n > arena_bytes - at)
-        fail(EKG_ENOMEM, "the group needs more than the " + std::to_string(arena_bytes >> 20) +
-                             " MiB static device workspace of the allocation-free entry point; use fewer "
-                             "requests per call or ekg_simulate_batch_device");
+    if (at > arena_bytes || n > arena_bytes - at) full();
     b.adopt(arena + at, n);
     arena_used = at + n;
+}
+
+void Workspace::full() const
+{
+    fail(EKG_ENOMEM, "the group needs more than the " + std::to_string(arena_bytes >> 20) +
+                             " MiB static device workspace of the allocation-free entry point; use fewer "
+                             "requests per call or ekg_simulate_batch_device");
 }
 
 void Ctx::bind() const { hip_check(hipSetDevice(device), "hipSetDevice"); }
@@ -955,10 +959,10 @@ ReqSizes req_sizes(const ReqSpec& r, bool mfma)
     return ReqSizes{mfma ? 0 : L.V + ekgk::MFMA_PAD, L.n_chunks, L.n_bricks, L.n_classes};
 }
 
-// Class sums of one request in the fixed workspace: a row per window piece
-// and class of the window, three sums per lead slot.  The launches divide
-// whatever that comes to among the 16-lead rows, so that the batch that fits
-// depends on this figure alone.
+// Least share of a request in the fixed workspace for its class sums and their
+// tables: a row per window piece and class of the window, three sums per lead
+// slot.  The batch that fits depends on it; the class sums take all that the
+// group's other buffers leave.
 int64_t fixed_class_bytes(const ReqSpec& r, int LP)
 {
     const EcgLayout& L = r.h->layout;
@@ -1196,7 +1200,15 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
         const ClassLines cl = class_lines(g);
         int64_t fixed = 0;
         for (const ReqSpec& r : g.reqs) fixed += fixed_class_bytes(r, LP);
-        int64_t cap = ws.arena ? fixed / LINE_BYTES : std::min(cl.all, GSUM_BYTES / LINE_BYTES);
+        int64_t cap = std::min(cl.all, GSUM_BYTES / LINE_BYTES);
+        if (ws.arena) {
+            // what is left of it after the tables and time grids below, each aligned
+            const size_t others = rd.size() * sizeof rd[0] + hdev.size() * sizeof hdev[0] + 7 * (B + 1) * 8 +
+                                  ws.h_tgrid.size() * 8 + ws.h_thl.size() * 4 + 3 * 256;
+            const int64_t room = (int64_t)ws.arena_bytes - (int64_t)((ws.arena_used + 255) & ~(size_t)255) - (int64_t)others;
+            if (room < fixed) ws.full();
+            cap = std::min(cap, (room - cl.table_bytes(1)) / LINE_BYTES);
+        }
         if (g.class_bytes >= 0) cap = std::min(cap, g.class_bytes / LINE_BYTES);
         cap = std::max<int64_t>(1, cap);
         ws.need(ws.gsum, (size_t)(cap * LINE_BYTES));

@@ -63,6 +63,7 @@ struct Workspace {
     size_t arena_bytes = 0, arena_used = 0;
     // reserve() for an owning workspace, a piece of the arena otherwise
     void need(DevBuf& b, size_t n);
+    [[noreturn]] void full() const;
     ~Workspace();
 };
 struct Ctx {

@@ -1,6 +1,7 @@
 """A group whose class sums need several launches (more than 256 MiB of them): the
 same bits as the requests alone, and a kernel time that covers every launch of
-the group."""
+the group.  The allocation-free entry point, whose class sums take what its workspace
+leaves: the same bits at few requests and at the most it takes."""
 import numpy as np
 import pytest
 
@@ -49,5 +50,30 @@ def test_rows_in_several_launches():
         for q in range(b, B, 12):
             assert np.array_equal(whole[q], alone)
     assert t_whole >= 0.85 * 2 * t_half
+    g.close()
+    ctx.close()
+
+
+def test_allocation_free_batches_up_to_the_limit():
+    import torch
+    ctx = E.Context(0)
+    n, L, T = 128, 12, 600
+    h = S.make_heart(n, seed=1)
+    g = E.Heart(ctx, h.layer, h.seed)
+    g.excite_delay(h.delay)
+    g.layout_info("3D4")
+    k8, p8 = _requests(n, L, 8, 90)
+    for B in (1, 8, 440):  # 440: the most requests of this shape
+        print(f"allocation-free batch of {B}", flush=True)
+        k = torch.from_numpy(np.resize(k8, (B,) + k8.shape[1:])).cuda()
+        p = torch.from_numpy(np.resize(p8, (B,) + p8.shape[1:])).cuda()
+        ref = torch.zeros((B, L, T), dtype=torch.float64, device="cuda")
+        got = torch.full((B, L, T), float("nan"), dtype=torch.float64, device="cuda")
+        args = (B, 3, L, "3D4", 0.0, float(T), 1.0)
+        g.simulate_batch_device(k.data_ptr(), p.data_ptr(), ref.data_ptr(), *args)
+        ctx.synchronize()
+        g.simulate_batch_device_noalloc(k.data_ptr(), p.data_ptr(), got.data_ptr(), *args)
+        ctx.synchronize()
+        assert torch.equal(got.view(torch.int64), ref.view(torch.int64))
     g.close()
     ctx.close()
