@@ -967,10 +967,10 @@ __global__ __launch_bounds__(1024) void ecg_chunk_kernel(
     // heart's activation) has no transition tiles and needs neither the voxels'
     // AP factors nor bounds.  Up to four leads that is worth a branch, and the
     // factors eP, eQ below one exponential in two lanes: 128 requests of a
-    // 24-layer heart with 2 leads from 100 ms 0.573 ms, 0.620 without.  With more
+    // 24-layer heart with 2 leads from 100 ms 0.567 ms, 0.609 without.  With more
     // leads the branch and the values it keeps in scalar registers (which spill
-    // in the lead field) cost 2% where every chunk has tiles: 64 x 12 leads
-    // on the 128^3 conduction-matrix heart 1.97 ms against 1.92.
+    // in the lead field) cost 5% where every chunk has tiles: 64 x 12 leads
+    // on the 128^3 conduction-matrix heart 1.90 ms against 1.81.
     constexpr bool LATE_AUX = LP == 4;
     const bool sat_ok = c1d < 0.0, skip_ok = kc.c1 < 0.0f && kc.skip != 0.0f;
     const bool trans =
@@ -1658,16 +1658,27 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
             }
         }
         __syncthreads();
-        double* const out = gsum + (sg.goff + (int64_t)rg * n_lines) * 16 + (t & 15);
-        const int split = reg.w >> 16, l1 = ext.w & 511, l2 = (ext.w >> 9) & 511, l3 = ext.w >> 18;
-        for (int i = t; i < (reg.w & 0xffff) * 16; i += 64 * CB_WAVES) {
-            const int ln = i >> 4, at = reg.z + ln - line0;
-            if ((unsigned)at >= (unsigned)n_lines) continue;  // a region that reaches past the launch's lines
-            const int p = (ln >= l1) + (ln >= l2) + (ln >= l3);
-            const int slot = ln - (ln >= l3 ? l3 : ln >= l2 ? l2 : ln >= l1 ? l1 : 0);
-            double v = 0.0;
-            for (int q = p; q < CB_WAVES; q += split) v += s_acc[q][slot][i & 15];
-            out[(int64_t)16 * at] = v;
+        const int64_t line = sg.goff + (int64_t)rg * n_lines + (reg.z - line0);
+        const int split = reg.w >> 16, nl = reg.w & 0xffff;
+        if (split == 1 && reg.z >= line0 && reg.z - line0 + nl <= n_lines) {
+            double* const out = gsum + line * 16;
+            for (int i = t; i < nl * 16; i += 64 * CB_WAVES) {
+                double v = 0.0;
+#pragma unroll
+                for (int q = 0; q < CB_WAVES; ++q) v += (&s_acc[q][0][0])[i];
+                out[i] = v;
+            }
+        } else {
+            const int l1 = ext.w & 511, l2 = (ext.w >> 9) & 511, l3 = ext.w >> 18;
+            for (int i = t; i < nl * 16; i += 64 * CB_WAVES) {
+                const int ln = i >> 4;
+                if ((unsigned)(reg.z - line0 + ln) >= (unsigned)n_lines) continue;  // past the launch's lines
+                const int p = (ln >= l1) + (ln >= l2) + (ln >= l3);
+                const int slot = ln - (ln >= l3 ? l3 : ln >= l2 ? l2 : ln >= l1 ? l1 : 0);
+                double v = 0.0;
+                for (int q = p; q < CB_WAVES; q += split) v += s_acc[q][slot][i & 15];
+                gsum[line * 16 + i] = v;
+            }
         }
         __syncthreads();
     }
