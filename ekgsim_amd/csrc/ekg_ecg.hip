@@ -1454,6 +1454,9 @@ __device__ __forceinline__ ScaleRange scale_range(float qz, float qy, float qx, 
     return r;
 }
 
+// PARTS: a launch with hearts whose waves divide the classes, or over a part of a
+// row's lines; the output that serves them costs the others 1 to 2%.
+template <bool PARTS>
 __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     const HeartDev* __restrict__ hearts, const ClassSeg* __restrict__ segs, int n_segs, const int* __restrict__ rowpos,
     const double* __restrict__ lead_pos, double* __restrict__ gsum, int line0, int line1, int reg0, int n_reg)
@@ -1476,7 +1479,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     // on XCD x with all its rows of 16 leads back to back, so that each region's
     // coefficients are fetched into one L2.  A block takes sg.per rows of a
     // region in turn (the chain of loads that starts a block, paid once).
-    const int nr = n_reg > 0 ? n_reg : sg.n_regions;
+    const int nr = PARTS && n_reg > 0 ? n_reg : sg.n_regions;
     const int local = (int)(blk - sg.block0), n8 = nr >> 3, ns = (sg.n_rg + sg.per - 1) / sg.per;
     int k, rg;
     if (local < 8 * n8 * ns) {
@@ -1489,7 +1492,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
         rg = q % ns * sg.per;
     }
     const int rg_end = rg + sg.per < sg.n_rg ? rg + sg.per : sg.n_rg;
-    k += reg0;
+    if constexpr (PARTS) k += reg0;
     const HeartDev& H = hearts[sg.heart];
     using ci32x4 = __attribute__((address_space(4))) const i32x4;
     using gi32x4 = __attribute__((address_space(1))) const i32x4;
@@ -1500,7 +1503,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     gi32x4* const pkt = (gi32x4*)H.cbox + lane;
     gi32x4* const ini = (gi32x4*)H.cinit + lane;
     const char* const coef = (const char*)H.ccoef;
-    const int n_lines = (line1 < H.n_lines ? line1 : H.n_lines) - line0;
+    const int n_lines = PARTS ? (line1 < H.n_lines ? line1 : H.n_lines) - line0 : H.n_lines;
     const int zq = lane >> 4;
     // electrode position offset of the lane's lead
     int po = ((gint*)rowpos)[16 * (sg.rg0 + rg) + (lane & 15)];
@@ -1658,26 +1661,25 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
             }
         }
         __syncthreads();
-        const int64_t line = sg.goff + (int64_t)rg * n_lines + (reg.z - line0);
-        const int split = reg.w >> 16, nl = reg.w & 0xffff;
-        if (split == 1 && reg.z >= line0 && reg.z - line0 + nl <= n_lines) {
-            double* const out = gsum + line * 16;
-            for (int i = t; i < nl * 16; i += 64 * CB_WAVES) {
+        if constexpr (!PARTS) {
+            double* out = gsum + (sg.goff + (int64_t)rg * n_lines + reg.z) * 16;
+            for (int i = t; i < (reg.w & 0xffff) * 16; i += 64 * CB_WAVES) {
                 double v = 0.0;
 #pragma unroll
                 for (int q = 0; q < CB_WAVES; ++q) v += (&s_acc[q][0][0])[i];
                 out[i] = v;
             }
         } else {
-            const int l1 = ext.w & 511, l2 = (ext.w >> 9) & 511, l3 = ext.w >> 18;
-            for (int i = t; i < nl * 16; i += 64 * CB_WAVES) {
-                const int ln = i >> 4;
-                if ((unsigned)(reg.z - line0 + ln) >= (unsigned)n_lines) continue;  // past the launch's lines
+            double* const out = gsum + (sg.goff + (int64_t)rg * n_lines) * 16 + (t & 15);
+            const int split = reg.w >> 16, l1 = ext.w & 511, l2 = (ext.w >> 9) & 511, l3 = ext.w >> 18;
+            for (int i = t; i < (reg.w & 0xffff) * 16; i += 64 * CB_WAVES) {
+                const int ln = i >> 4, at = reg.z + ln - line0;
+                if ((unsigned)at >= (unsigned)n_lines) continue;  // past the launch's lines
                 const int p = (ln >= l1) + (ln >= l2) + (ln >= l3);
                 const int slot = ln - (ln >= l3 ? l3 : ln >= l2 ? l2 : ln >= l1 ? l1 : 0);
                 double v = 0.0;
                 for (int q = p; q < CB_WAVES; q += split) v += s_acc[q][slot][i & 15];
-                gsum[line * 16 + i] = v;
+                out[(int64_t)16 * at] = v;
             }
         }
         __syncthreads();
@@ -2028,7 +2030,8 @@ hipError_t launch_class_boxes(const GroupArgs& a, const ClassLaunch& c, hipStrea
 {
     if (c.blocks < 0 || c.blocks > 0x7fffffffLL || c.n_segs < 1) return hipErrorInvalidValue;
     if (c.blocks == 0) return hipSuccess;  // hearts without class cells: their sums are zero
-    hipLaunchKernelGGL(ecg_class_box_kernel, dim3((unsigned)c.blocks), dim3(64 * CB_WAVES), 0, s, a.hearts,
+    hipLaunchKernelGGL(c.parts ? ecg_class_box_kernel<true> : ecg_class_box_kernel<false>, dim3((unsigned)c.blocks),
+                       dim3(64 * CB_WAVES), 0, s, a.hearts,
                        a.segs + c.seg0, c.n_segs, a.rowpos, a.lead_pos, a.gsum, c.l0, c.l1, c.reg0, c.n_reg);
     return hipGetLastError();
 }
@@ -2104,7 +2107,8 @@ void prime_kernels()
 {
     hipFuncAttributes at;
     (void)hipFuncGetAttributes(&at, (const void*)ap_tables_kernel);
-    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel);
+    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel<false>);
+    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel<true>);
     prime_lp<4>(at);
     prime_lp<8>(at);
     prime_lp<12>(at);

@@ -938,6 +938,7 @@ void ensure_cells(Heart& h, int nhood)
     L.n_centries[nhood] = n_entries;
     L.n_cpieces[nhood] = (int)n_pieces;
     L.n_lines[nhood] = (int)lines.size();
+    L.class_parts[nhood] = split;
     L.h_region_line[nhood].clear();
     for (const int4& r : regions) L.h_region_line[nhood].push_back(r.z);
     L.h_region_line[nhood].push_back((int)lines.size());
@@ -1242,7 +1243,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
                         if (cut - l0 >= cap / 2 && cut > l0) l1 = cut;
                         const int reg0 = (int)(std::upper_bound(rl.begin(), rl.end(), (int)l0) - rl.begin()) - 1;
                         const int reg1 = (int)(std::lower_bound(rl.begin(), rl.end(), (int)l1) - rl.begin());
-                        launches.push_back({(int)segs.size(), 1, rg, 1, (int)l0, (int)l1, reg0, reg1 - reg0, reg1 - reg0});
+                        launches.push_back({(int)segs.size(), 1, rg, 1, (int)l0, (int)l1, reg0, reg1 - reg0, reg1 - reg0, 1});
                     }
                     segs.push_back(ekgk::ClassSeg{rg, 1, hl.n_regions[g.nhood], rd[r].heart, 1, 0, block0, 0});
                     rgseg.push_back((int)segs.size() - 1);
@@ -1267,6 +1268,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
                 block0 += nblk;
                 la.blocks += nblk;
                 ++la.n_segs;
+                if (hl.class_parts[g.nhood] > 1) la.parts = 1;
                 la.n_rg += n;
                 used += n * lines;
                 rg += n;

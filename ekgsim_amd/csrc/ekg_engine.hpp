@@ -119,6 +119,7 @@ struct EcgLayout {
     int64_t n_ccells[4] = {0, 0, 0, 0}, n_centries[4] = {0, 0, 0, 0};
     int n_cpieces[4] = {0, 0, 0, 0}, n_lines[4] = {0, 0, 0, 0}, n_regions[4] = {0, 0, 0, 0};
     std::vector<int> h_region_line[4];  // first line of each region, then their end
+    int class_parts[4] = {1, 1, 1, 1};  // parts of a region's classes
     DevBuf cregion[4], cbox[4], cinit[4], ccoef[4], cmask[4], cs_off[4], cs_line[4];
     std::vector<int> h_layer_chunk;
     std::vector<double> h_layer_t0;

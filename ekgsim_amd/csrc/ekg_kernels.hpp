@@ -96,7 +96,7 @@ struct HeartDev {
 // One request of a launch group.  Offsets index the group's packed arrays.
 struct ReqDev {
     int heart, L, nl, T, Tn, Tp, n_tiles;
-    int bt_shift;     // log2 of the bound tiles of the chunk bounds and prefix tables (16 or 64 steps)
+    int bt_shift;     // log2 of the bound tiles of the chunk bounds and prefix tables (8 or 64 steps)
     int64_t k_off;    // layer_k[k_off + 9*(l-1) + q]
     int64_t pos_off;  // lead_pos[pos_off + 3*i + c]
     int64_t ecg_off;  // ecg[ecg_off + i*T + j]
@@ -125,6 +125,7 @@ struct ClassLaunch {
     int seg0, n_segs, rg0, n_rg;
     int l0 = 0, l1 = 0x7fffffff, reg0 = 0, n_reg = 0;  // n_reg 0: all lines and regions
     int64_t blocks = 0;
+    int64_t parts = 0;         // 1: such lines, or a heart whose regions have parts
 };
 
 // A launch group: requests of any hearts, lead counts and time grids that
