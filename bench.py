@@ -102,7 +102,7 @@ NAIVE_LANE_CYCLES, LANE_PEAK = 38, 256 * 64 * 2.4e9
 # 256 MiB calibration copy: with activation classes
 # (profiles/ecg_class_box_kernel_128cubed_batch256_hbm_traffic.md) and
 # without (profiles/ecg_chunk_kernel_128cubed_batch256_hbm_traffic.md).
-TRAFFIC_BYTES = {"ecg_class_box_kernel": 230056000, "ecg_chunk_kernel": 1131874216}
+TRAFFIC_BYTES = {"ecg_class_box_kernel": 195717051, "ecg_chunk_kernel": 1131874216}
 # Issue-pipe occupancy of the dominant kernel on this workload, from one
 # rocprofv3 --pmc pass (SQ_VALU_MFMA_BUSY_CYCLES, SQ_INSTS_VALU minus the MFMA
 # instructions at 4 cycles each, SQ_VALU_MFMA_COEXEC_CYCLES, GRBM_GUI_ACTIVE)
@@ -110,7 +110,7 @@ TRAFFIC_BYTES = {"ecg_class_box_kernel": 230056000, "ecg_chunk_kernel": 11318742
 # and profiles/ecg_chunk_kernel_128cubed_batch256_pipes.md.  The sum
 # less the overlap is the fraction of the kernel's cycles spent issuing; FP64
 # products never overlap the vector ALU (chunk kernel), int8 ones do.
-PIPES = {"ecg_class_box_kernel": {"mfma_busy": 0.181, "valu_issue": 0.645, "coexec": 0.070},
+PIPES = {"ecg_class_box_kernel": {"mfma_busy": 0.188, "valu_issue": 0.662, "coexec": 0.074},
          "ecg_chunk_kernel": {"mfma_busy": 0.116, "valu_issue": 0.806, "coexec": 0.0}}
 
 

@@ -1391,7 +1391,7 @@ __global__ void ecg_reduce_parts_kernel(const HeartDev* __restrict__ hearts, con
 // the groups of waves of all parts the boxes: regions of 96 classes would hold one
 // or two boxes there (figures at class_cut).  The cut into regions and the order
 // depend on the heart only, so a request's bits do not depend on its batch.
-// Measured per 256 x 12 launch on the 128^3 heart: 0.83 ms (vector instructions
+// Measured per 256 x 12 launch on the 128^3 heart: 0.80 ms (vector instructions
 // 0.52 and matrix products 0.15 of it), against 1.37 ms with the weights
 // evaluated per window of six classes and FP64 products; 16 x 12 on the 256^3 heart
 // 0.35 against 0.69 ms.  Regions of 64 classes instead of 96: 0.97 ms (a block's
