@@ -1454,15 +1454,22 @@ __device__ __forceinline__ ScaleRange scale_range(float qz, float qy, float qx, 
     return r;
 }
 
-// PARTS: a launch with hearts whose waves divide the classes, or over a part of a
-// row's lines; the output that serves them costs the others 1 to 2%.
-template <bool PARTS>
+// MODE 1: a launch with hearts whose waves divide the classes in two parts, or over a part
+// of a row's lines; the output that serves them costs the others (MODE 0) 1 to 2%.
+// MODE 2: hearts with four parts.  All waves of a block take the same box then, each forms
+// the weights of one sub-brick, and the four go round in LDS.  With every wave
+// forming all of them they were half of the vector instructions: 64 requests of 12 leads on a
+// 24-layer 112^3 heart 936 us, 872 so (one 138 and 125; 256 3,337 and 3,116).
+template <int MODE>
 __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     const HeartDev* __restrict__ hearts, const ClassSeg* __restrict__ segs, int n_segs, const int* __restrict__ rowpos,
     const double* __restrict__ lead_pos, double* __restrict__ gsum, int line0, int line1, int reg0, int n_reg)
 {
-    __shared__ double s_acc[CB_WAVES][CB_SLOTS + 1][16];  // last row: classes past a tile's end
+    constexpr bool PARTS = MODE > 0, SHARED = MODE == 2;
+    constexpr int SLOTS = SHARED ? CB_SLOTS4 : CB_SLOTS;
+    __shared__ double s_acc[CB_WAVES][SLOTS + 1][16];  // last row: classes past a tile's end
     __shared__ i32x4 s_init[CB_WAVES][64];
+    __shared__ i32x4 s_w[SHARED ? 4 : 1][4][64];       // [sub-brick][limb]: a box's weights
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int64_t blk = segs[0].block0 + blockIdx.x;
@@ -1510,7 +1517,7 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
     for (; rg < rg_end; ++rg) {
         const double p0 = ((gf64*)lead_pos)[po], p1 = ((gf64*)lead_pos)[po + 1], p2 = ((gf64*)lead_pos)[po + 2];
         if (rg + 1 < rg_end) po = ((gint*)rowpos)[16 * (sg.rg0 + rg + 1) + (lane & 15)];
-        for (int i = lane; i < (CB_SLOTS + 1) * 16; i += 64) (&s_acc[w][0][0])[i] = 0.0;
+        for (int i = lane; i < (SLOTS + 1) * 16; i += 64) (&s_acc[w][0][0])[i] = 0.0;
 
         // One scale for the whole region where every lead of the row allows it
         // (most regions: a lead at least about 10 voxels off), else per box.
@@ -1535,8 +1542,8 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
             wave_lds_fence();      // the box before: its reads of s_init and its sums in s_acc
             s_init[w][lane] = nin;
             wave_lds_fence();
-            // lane 16: {tiles, rows (4 sub-brick + y) in use, 0, 0}; lane 17: first cell + 1
-            const int nt = __builtin_amdgcn_readlane(tr.x, 16), rows = __builtin_amdgcn_readlane(tr.y, 16);
+            // lane 16: {tiles, rows (4 sub-brick + y) in use, in use by any part, 0}; lane 17: first cell + 1
+            const int nt = __builtin_amdgcn_readlane(tr.x, 16), rows = __builtin_amdgcn_readlane(SHARED ? tr.z : tr.y, 16);
             // electrode relative to the box's first cell
             double qz = p0 - (double)__builtin_amdgcn_readlane(tr.x, 17), qy = p1 - (double)__builtin_amdgcn_readlane(tr.y, 17),
                    qx = p2 - (double)__builtin_amdgcn_readlane(tr.z, 17);
@@ -1576,12 +1583,14 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                 // |e|^2 x 4^-m = X[x] + Y[y], formed in each pass (the pin keeps them
                 // out of the registers of the tile loop below)
                 asm volatile("" : "+v"(qz), "+v"(qy), "+v"(qx));
-                double X[8], Y[8];
+                constexpr int NX = SHARED ? 4 : 8;  // of one sub-brick, or of all
+                double X[NX], Y[NX];
                 const double sz = qz * st, sy = qy * st, sx = qx * st;
                 const double tz = __builtin_fma((double)-zq, st, sz), Z = tz * tz;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const double tx = __builtin_fma((double)-i, st, sx), ty = __builtin_fma((double)-i, st, sy);
+                for (int i = 0; i < NX; ++i) {
+                    const int ix = SHARED ? i + 4 * (w & 1) : i, iy = SHARED ? i + 4 * (w >> 1) : i;
+                    const double tx = __builtin_fma((double)-ix, st, sx), ty = __builtin_fma((double)-iy, st, sy);
                     X[i] = tx * tx;
                     Y[i] = __builtin_fma(ty, ty, Z);
                 }
@@ -1604,14 +1613,16 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                 load_tile();
                 i32x4 W[4][4];  // [sub-brick][limb]: bytes 4 y + x
 #pragma unroll
-                for (int sb = 0; sb < 4; ++sb) {
+                for (int sb = 0; sb < (SHARED ? 1 : 4); ++sb) {
+                    const int rw = SHARED ? rows >> (4 * w) : rows >> (4 * sb);
 #pragma unroll
                     for (int y = 0; y < 4; ++y) {
-                        if (!((rows >> (4 * sb + y)) & 1)) continue;  // only zero coefficients
+                        if (!((rw >> y) & 1)) continue;  // only zero coefficients
                         float s[4];
 #pragma unroll
                         for (int x = 0; x < 4; ++x) {
-                            const float r = __builtin_amdgcn_rsqf((float)(X[4 * (sb & 1) + x] + Y[4 * (sb >> 1) + y]));
+                            const float r = __builtin_amdgcn_rsqf(
+                                (float)(X[SHARED ? x : 4 * (sb & 1) + x] + Y[SHARED ? y : 4 * (sb >> 1) + y]));
                             s[x] = r * r * r;
                         }
                         if (hot) {
@@ -1629,7 +1640,16 @@ __global__ __launch_bounds__(64 * CB_WAVES, 3) void ecg_class_box_kernel(
                 }
                 // rows left out: whatever their registers hold, it counts as a value
 #pragma unroll
-                for (int i = 0; i < 16; ++i) asm("" : "+v"((&W[0][0])[i]));
+                for (int i = 0; i < (SHARED ? 4 : 16); ++i) asm("" : "+v"((&W[0][0])[i]));
+                if constexpr (SHARED) {
+                    // the four waves have the same boxes and passes, so all come here
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) s_w[w][j][lane] = W[0][j];
+                    __syncthreads();
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) (&W[0][0])[i] = (&s_w[0][0][0])[64 * i + lane];
+                    __syncthreads();
+                }
                 const double cz = qz * sc, cy = qy * sc, cx = qx * sc;
                 for (;;) {
                     const i32x4 c0 = s_init[w][4 * (ti & 15) + zq];
@@ -2030,8 +2050,10 @@ hipError_t launch_class_boxes(const GroupArgs& a, const ClassLaunch& c, hipStrea
 {
     if (c.blocks < 0 || c.blocks > 0x7fffffffLL || c.n_segs < 1) return hipErrorInvalidValue;
     if (c.blocks == 0) return hipSuccess;  // hearts without class cells: their sums are zero
-    hipLaunchKernelGGL(c.parts ? ecg_class_box_kernel<true> : ecg_class_box_kernel<false>, dim3((unsigned)c.blocks),
-                       dim3(64 * CB_WAVES), 0, s, a.hearts,
+    hipLaunchKernelGGL(c.parts == 2   ? ecg_class_box_kernel<2>
+                       : c.parts == 1 ? ecg_class_box_kernel<1>
+                                      : ecg_class_box_kernel<0>,
+                       dim3((unsigned)c.blocks), dim3(64 * CB_WAVES), 0, s, a.hearts,
                        a.segs + c.seg0, c.n_segs, a.rowpos, a.lead_pos, a.gsum, c.l0, c.l1, c.reg0, c.n_reg);
     return hipGetLastError();
 }
@@ -2107,8 +2129,9 @@ void prime_kernels()
 {
     hipFuncAttributes at;
     (void)hipFuncGetAttributes(&at, (const void*)ap_tables_kernel);
-    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel<false>);
-    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel<true>);
+    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel<0>);
+    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel<1>);
+    (void)hipFuncGetAttributes(&at, (const void*)ecg_class_box_kernel<2>);
     prime_lp<4>(at);
     prime_lp<8>(at);
     prime_lp<12>(at);

@@ -595,28 +595,30 @@ namespace {
 // With few classes to a box a region holds boxes enough for its block's four
 // waves, each for all of the classes.  With many, one or two boxes fill the region's
 // slots, which leaves waves idle and a line of sums for almost every class of a
-// box; so the waves divide the classes, at the price of a box's weights once a
-// part, and the region holds as many times the classes.  Measured on
+// box; so the waves divide the classes, and the region holds as many times the
+// classes.  In two parts each wave forms the weights of its boxes, so a box's weights
+// are formed twice; in four all waves take the same box and share its weights.  Measured on
 // integer-delay hearts, us for 1 / 64 / 256 requests of 12 leads and 64 steps:
-//   classes a box   1 part               2 parts              4 parts
-//   112^3, 27       100 / 330 / 1,165     89 / 368 / 1,288    107 / 515 / 1,788
-//   144^3, 34       124 / 889 / -        104 / 758 / -        114 / 1,043 / -
-//   112^3, 37       100 / 482 / 1,786    100 / 422 / 1,474    121 / 561 / 2,001
-//   144^3, 43       145 / 1,245 / 4,816  123 / 795 / 2,909    136 / 1,094 / 3,957
-//   112^3, 62       120 / 1,151 / 4,426  119 / 691 / 2,432    152 / 723 / 2,589
-//   144^3, 73       201 / 3,710 / 14,434 161 / 1,568 / 5,981  182 / 1,436 / 5,230
-// Larger regions have fewer lines, smaller ones more blocks for a lone request:
-// 80^3 with 50 classes a box and two parts, 92 / 281 / 921 us with 8 boxes,
-// 92 / 277 / 898 with 12, 98 / 267 / 830 with 16.
+//   classes a box   1 part                 2 parts              4 parts
+//   112^3, 27       100 / 330 / 1,165       89 / 368 / 1,288     87 / 401 / 1,358
+//   112^3, 37       100 / 482 / 1,786      100 / 422 / 1,474     94 / 460 / 1,663
+//   144^3, 43       145 / 1,245 / 4,816    123 / 795 / 2,909    113 / 925 / 3,330
+//   112^3, 62       120 / 1,151 / 4,426    119 / 691 / 2,432    114 / 666 / 2,393
+//   144^3, 73       201 / 3,710 / 14,434   161 / 1,568 / 5,981  147 / 1,421 / 5,301
+// (34 classes at 144^3: 124 / 889 / - in one part, 104 / 758 / - in two).  Larger
+// regions have fewer lines, smaller ones more blocks for a lone request: 80^3 with
+// 50 classes a box and two parts, 92 / 281 / 921 us with 8 boxes, 92 / 277 / 898 with 12,
+// 98 / 267 / 830 with 16; 112^3 with 78 and four parts 125 / 900 / 3,334 with 4, 125 / 872 /
+// 3,116 with 8, 140 / 916 / 3,292 with 16.
 struct Cut {
     int split, boxes;
 };
 
 Cut class_cut(int64_t pairs, int64_t boxes)
 {
-    const int split = pairs <= 33 * boxes ? 1 : pairs <= 70 * boxes ? 2 : 4;
-    if (split == 1) return {1, (int)std::min<int64_t>(64, std::max<int64_t>(4, (boxes / 64 + 3) / 4 * 4))};
-    return {split, (int)std::min<int64_t>(16, std::max<int64_t>(split == 2 ? 12 : 8, boxes / 192))};
+    if (pairs <= 33 * boxes) return {1, (int)std::min<int64_t>(64, std::max<int64_t>(4, (boxes / 64 + 3) / 4 * 4))};
+    if (pairs <= 60 * boxes) return {2, (int)std::min<int64_t>(16, std::max<int64_t>(12, boxes / 192))};
+    return {4, 8};
 }
 
 }  // namespace
@@ -725,7 +727,7 @@ void ensure_cells(Heart& h, int nhood)
     std::vector<int8_t> coef;                 // 1024 per block
     std::vector<uint64_t> mask;               // 4 per listed box
     std::vector<std::pair<int, int>> lines;   // (class, line)
-    // A region's classes are divided over `split` parts with CB_SLOTS slots each:
+    // A region's classes are divided over `split` parts with CB_SLOTS (or CB_SLOTS4) slots each:
     // wave w of a block adds the classes of part w % split, of every
     // (CB_WAVES / split)-th box.
     int64_t pairs = 0;  // (box, class)
@@ -734,6 +736,7 @@ void ensure_cells(Heart& h, int nhood)
     const Cut cut = class_cut(pairs, (int64_t)order.size());
     const int split = cut.split, target = cut.boxes;
     const int groups = ekgk::CB_WAVES / split;
+    const int slots_part = split == 4 ? ekgk::CB_SLOTS4 : CB_SLOTS;
     std::vector<int> slot_of(L.n_classes, -1);     // part << 8 | slot in the current region
     std::vector<std::vector<int>> slot_cls(split);  // the region's classes by part and slot
     std::vector<int> cost;  // per item (box listing, one packet a part) of the current region
@@ -797,7 +800,7 @@ void ensure_cells(Heart& h, int nhood)
             if (slot_of[cls[c1]] < 0) {
                 p = -1;
                 for (int q = 0; q < split; ++q)
-                    if (slot_cls[q].size() < (size_t)CB_SLOTS && (p < 0 || part[q].size() < part[p].size())) p = q;
+                    if (slot_cls[q].size() < (size_t)slots_part && (p < 0 || part[q].size() < part[p].size())) p = q;
             }
             if (p >= 0 && part[p].size() == BOX_CLASSES) break;
             if (p < 0) {
@@ -847,7 +850,8 @@ void ensure_cells(Heart& h, int nhood)
                 ext.push_back(int4{0xffff, 0xffff, 0xffff, 0});
                 take(c0, c1);
             }
-            int item_cost = 0;
+            int item_cost = 0, item_rows = 0;
+            const size_t item = pkt.size();
             const int o[3] = {bz * BOX_Z + 1, by * BOX_Y + 1, bx * BOX_X + 1};
             for (const std::vector<size_t>& pc : part) {
                 const size_t blk0 = coef.size() / 1024;
@@ -862,7 +866,7 @@ void ensure_cells(Heart& h, int nhood)
                     unsigned slots = 0;
                     int subs = 0;
                     for (size_t q = q0; q < q0 + 4; ++q) {
-                        slots |= (unsigned)(q < q1 ? slot_of[cls[pc[q]]] & 255 : CB_SLOTS) << (8 * (q - q0));
+                        slots |= (unsigned)(q < q1 ? slot_of[cls[pc[q]]] & 255 : slots_part) << (8 * (q - q0));
                         if (q < q1) subs |= cls_sub[pc[q]];
                     }
                     if (coef.size() / 1024 > 0x7ffffff0u) fail(EKG_EINVAL, "too many class cells");
@@ -887,6 +891,7 @@ void ensure_cells(Heart& h, int nhood)
                         }
                 }
                 pkt[pk + 16] = int4{n_tile, used, 0, 0};
+                item_rows |= used;
                 pkt[pk + 17] = int4{o[0], o[1], o[2], 0};
                 // cycles of a box, roughly: 34 a weight of 64 lanes, 64 a block's
                 // four products, 180 a tile's flush
@@ -895,6 +900,7 @@ void ensure_cells(Heart& h, int nhood)
                 ++n_box;
                 mask.insert(mask.end(), bm, bm + 4);
             }
+            for (int p = 0; p < split; ++p) pkt[item + 64 * p + 16].z = item_rows;
             cost.push_back(item_cost);
             const int len[3] = {BOX_Z, BOX_Y, BOX_X};
             int* e = &ext.back().x;
@@ -1243,7 +1249,8 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
                         if (cut - l0 >= cap / 2 && cut > l0) l1 = cut;
                         const int reg0 = (int)(std::upper_bound(rl.begin(), rl.end(), (int)l0) - rl.begin()) - 1;
                         const int reg1 = (int)(std::lower_bound(rl.begin(), rl.end(), (int)l1) - rl.begin());
-                        launches.push_back({(int)segs.size(), 1, rg, 1, (int)l0, (int)l1, reg0, reg1 - reg0, reg1 - reg0, 1});
+                        launches.push_back({(int)segs.size(), 1, rg, 1, (int)l0, (int)l1, reg0, reg1 - reg0, reg1 - reg0,
+                                            hl.class_parts[g.nhood] == 4 ? 2 : 1});
                     }
                     segs.push_back(ekgk::ClassSeg{rg, 1, hl.n_regions[g.nhood], rd[r].heart, 1, 0, block0, 0});
                     rgseg.push_back((int)segs.size() - 1);
@@ -1252,7 +1259,8 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
                     ++rg;
                     continue;
                 }
-                if (used + lines > cap || launches.back().n_rg >= 65535) {
+                const bool four = hl.class_parts[g.nhood] == 4;  // a kernel instance of its own
+                if (used + lines > cap || launches.back().n_rg >= 65535 || four != (launches.back().parts == 2)) {
                     launches.push_back({(int)segs.size(), 0, rg, 0});
                     used = 0;
                 }
@@ -1268,7 +1276,7 @@ void enqueue_group(Ctx& ctx, GroupPlan& g, Workspace& ws, hipStream_t stream, co
                 block0 += nblk;
                 la.blocks += nblk;
                 ++la.n_segs;
-                if (hl.class_parts[g.nhood] > 1) la.parts = 1;
+                if (hl.class_parts[g.nhood] > 1) la.parts = four ? 2 : 1;
                 la.n_rg += n;
                 used += n * lines;
                 rg += n;

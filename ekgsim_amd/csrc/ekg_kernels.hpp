@@ -27,6 +27,8 @@ constexpr int BT_SHIFT_VALU = 6;
 // region (LDS rows of 16 leads per wave: 12.4 KB, so that three blocks share a CU).
 constexpr int CB_WAVES = 4;
 constexpr int CB_SLOTS = 96;
+// Classes of each of four parts: the waves' shared weights take the LDS of the other 32.
+constexpr int CB_SLOTS4 = 64;
 
 // ---- excitation sequence ---------------------------------------------------
 
@@ -125,7 +127,7 @@ struct ClassLaunch {
     int seg0, n_segs, rg0, n_rg;
     int l0 = 0, l1 = 0x7fffffff, reg0 = 0, n_reg = 0;  // n_reg 0: all lines and regions
     int64_t blocks = 0;
-    int64_t parts = 0;         // 1: such lines, or a heart whose regions have parts
+    int64_t parts = 0;         // 1: such lines, or a heart whose regions have two parts; 2: hearts with four
 };
 
 // A launch group: requests of any hearts, lead counts and time grids that
