@@ -583,7 +583,7 @@ void ensure_layout(Heart& h, bool mfma)
 //    times the sum of their coefficients.
 //  * Consecutive boxes form regions, whose class sums a block keeps in LDS: at
 //    most CB_SLOTS classes, or on hearts with many classes to a box CB_SLOTS for each
-//    of 2 or 4 parts that the waves divide (class_cut); a box with more classes is
+//    of 2 parts or CB_SLOTS4 of 4 that the waves divide (class_cut); a box with more classes is
 //    listed again with the rest.  With parts, a box is listed once a part, with the
 //    part's classes.
 //    Each (region, class) has a line of sums, listed per class in order.
